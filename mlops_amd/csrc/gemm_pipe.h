@@ -191,4 +191,43 @@ __device__ __forceinline__ int tile_of(int round, int block, int grid) {
   return round * grid + block;
 }
 
+// x / d for the divisor d encoded by row_div_magic (s == 0: d = 1): the
+// round-down multiply-high method for unsigned division by an invariant
+// integer (Granlund and Montgomery, PLDI 1994), with a 33-bit multiplier
+// 2^32 + m, exact for every 32-bit x.
+__device__ __forceinline__ uint32_t div_rows(uint32_t x, uint32_t m, int s) {
+  const uint32_t t = __umulhi(x, m);
+  const uint32_t q = (t + ((x - t) >> 1)) >> (s > 0 ? s - 1 : 0);
+  return s == 0 ? x : q;  // a select: no branch around the LDS reads it feeds
+}
+
+// (m, s) for div_rows: s = ceil(log2 d), m = floor(2^32 (2^s - d) / d) + 1
+// for d >= 2; (0, 0) for d = 1.
+struct RowDiv {
+  uint32_t m;
+  int s;
+};
+inline RowDiv row_div_magic(int d) {
+  if (d <= 1) return {0u, 0};
+  int s = 0;
+  while ((1 << s) < d) ++s;
+  const uint64_t m = (((uint64_t)1 << 32) * (uint64_t)((1 << s) - d)) / (uint64_t)d + 1;
+  return {(uint32_t)m, s};
+}
+
+// Compute units of the current device (cached; host side).
+inline int cu_count() {
+  static int cus[64] = {0};
+  int dev = 0;
+  hipGetDevice(&dev);
+  if (dev < 0 || dev >= 64) dev = 0;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 }  // namespace pipe

@@ -5,6 +5,15 @@
 
 using namespace pipe;
 
+// gemm_tile.hip: the launch on smaller tiles; returns 1 outside its range.
+int mi355x_gemm_tile_launch(const uint8_t* a, const float* a_scale, int rows, const uint8_t* w,
+                            const float* w_scale, int w_scale_t, int experts, int n, int k,
+                            const int32_t* offsets, int interleave, const void* addend,
+                            const void* lora_z, const void* lora_b, int lora_rank, void* out,
+                            const int32_t* a_rows, int a_rows_div, bool row, bool kmajor,
+                            void* stream);
+bool mi355x_gemm_tile_serves(int rows, int experts, int n);
+
 namespace {
 
 constexpr int kMaxExperts = 512;
@@ -81,16 +90,6 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 // 128 K rows of 256 bytes and the B fragments read with ds_read_b64_tr_b8;
 // the MFMA columns are then the tile's columns in order, so the epilogue
 // regroups each row's values through LDS into 8-column stores.
-// x / d for the divisor d encoded by row_div_magic (s == 0: d = 1): the
-// round-down multiply-high method for unsigned division by an invariant
-// integer (Granlund and Montgomery, PLDI 1994), with a 33-bit multiplier
-// 2^32 + m, exact for every 32-bit x.
-__device__ __forceinline__ uint32_t div_rows(uint32_t x, uint32_t m, int s) {
-  const uint32_t t = __umulhi(x, m);
-  const uint32_t q = (t + ((x - t) >> 1)) >> (s > 0 ? s - 1 : 0);
-  return s == 0 ? x : q;  // a select: no branch around the LDS reads it feeds
-}
-
 // MFMA block of a K step at which waves 4-7 issue the next step's copies.
 constexpr int kLateIssueBlock = 1;
 
@@ -570,20 +569,6 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
   }
 }
 
-int cu_count() {
-  static int cus[64] = {0};
-  int dev = 0;
-  hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64) dev = 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 }  // namespace
 
 // Tile order by the size of one expert's weight (N x K bytes). Up to a few
@@ -605,20 +590,6 @@ Order tile_order(int n, int k) {
 }
 }  // namespace
 
-// (m, s) for div_rows: s = ceil(log2 d), m = floor(2^32 (2^s - d) / d) + 1
-// for d >= 2; (0, 0) for d = 1.
-struct RowDiv {
-  uint32_t m;
-  int s;
-};
-RowDiv row_div_magic(int d) {
-  if (d <= 1) return {0u, 0};
-  int s = 0;
-  while ((1 << s) < d) ++s;
-  const uint64_t m = (((uint64_t)1 << 32) * (uint64_t)((1 << s) - d)) / (uint64_t)d + 1;
-  return {(uint32_t)m, s};
-}
-
 // Launches the pipelined kernel; returns 1 if the shape is not its form
 // (N % 256 != 0), in which case the caller uses the general kernel.
 int mi355x_gemm_v2_launch(const uint8_t* a, const float* a_scale, int rows, const uint8_t* w,
@@ -627,6 +598,15 @@ int mi355x_gemm_v2_launch(const uint8_t* a, const float* a_scale, int rows, cons
                           uint8_t* act_q, float* act_scales, float limit, const void* lora_z,
                           const void* lora_b, int lora_rank, void* stream,
                           const int32_t* a_rows, int a_total, int a_rows_div) {
+  if (act_q == nullptr) {
+    const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, w_scale_t, experts, n,
+                                              k, offsets, interleave, addend, lora_z, lora_b,
+                                              lora_rank, out, a_rows, a_rows_div, false, false,
+                                              stream);
+    if (small <= 0) return small;
+  } else if (mi355x_gemm_tile_serves(rows, experts, n)) {
+    return 1;  // the caller runs the GEMM, then the SwiGLU pass: the same bytes
+  }
   if (n % BN != 0 || experts > kMaxExperts || (interleave && (n / 2) % 128 != 0)) return 1;
   const RowDiv div = row_div_magic(a_rows_div);
   const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);
@@ -662,6 +642,10 @@ int mi355x_gemm_v2_kmajor_launch(const uint8_t* a, const float* a_scale, int row
                                  const uint8_t* w, const float* w_scale, int experts, int n, int k,
                                  const int32_t* offsets, void* out, void* stream,
                                  const int32_t* a_rows, int a_total, int a_rows_div) {
+  const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, 1, experts, n, k,
+                                            offsets, 0, nullptr, nullptr, nullptr, 0, out, a_rows,
+                                            a_rows_div, false, true, stream);
+  if (small <= 0) return small;
   if (n % BN != 0 || experts > kMaxExperts) return 1;
   const RowDiv div = row_div_magic(a_rows_div);
   const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);
@@ -687,6 +671,10 @@ int mi355x_gemm_v2_rowwise_launch(const uint8_t* a, const float* a_scale, int ro
                                   int k, const int32_t* offsets, const void* lora_z,
                                   const void* lora_b, int lora_rank, void* out, void* stream,
                                   const int32_t* a_rows, int a_total, int a_rows_div) {
+  const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, 0, experts, n, k,
+                                            offsets, 0, nullptr, lora_z, lora_b, lora_rank, out,
+                                            a_rows, a_rows_div, true, false, stream);
+  if (small <= 0) return small;
   if (n % BN != 0 || experts > kMaxExperts) return 1;
   const RowDiv div = row_div_magic(a_rows_div);
   const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);

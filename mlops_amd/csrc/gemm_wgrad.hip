@@ -229,20 +229,6 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
   }
 }
 
-int cu_count() {
-  static int cus[64] = {0};
-  int dev = 0;
-  hipGetDevice(&dev);
-  if (dev < 0 || dev >= 64) dev = 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 }  // namespace
 
 // Launches the pipelined kernel; returns 1 if the shape is not its form

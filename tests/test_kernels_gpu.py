@@ -362,6 +362,78 @@ def test_grouped_gemm_matches_fp64(device, case):
     assert worst_cell_rel(out, want, offsets.tolist()) < 1e-2
 
 
+# Row counts and N that reach each tile size of the grouped GEMM: 64-row tiles
+# (few rows a group; 1 to 3 K steps, shorter than the copy pipeline), 128-row
+# tiles (129..160 rows a group), the 256 x 256 tiles, and 256 x 128 tiles (N an
+# odd multiple of 128 over many row blocks).
+TILE_CASES = [
+    ([1, 63, 64, 65, 0, 17], 512, 128),
+    ([1, 63, 64, 65, 0, 17], 768, 256),
+    ([1, 63, 64, 65, 0, 17], 384, 384),
+    ([3], 256, 1024),
+    ([129, 160, 256, 1, 250], 512, 128),
+    ([129, 160, 256, 1, 250], 256, 640),
+    ([129, 160, 256, 1, 250], 384, 384),
+    ([300, 511, 0, 900], 4096, 256),
+    ([300, 511, 0, 900], 12416, 128),
+]
+
+
+@pytest.mark.parametrize("counts,n,k", TILE_CASES)
+def test_grouped_gemm_forms_at_every_tile_size(device, counts, n, k):
+    """Every operand form at each tile size against the fp64 product of the
+    dequantized operands. Bound: one bf16 rounding of the result is 2^-9 of
+    each element, fp32 sums of K / 128 block partials add 1e-6, and a 128
+    column cell averages them: 4e-3 is twice the worst rounding. Forms that
+    read the same operands another way are bitwise equal."""
+    for options in (dict(), dict(transposed=True), dict(interleave=True), dict(addend=True),
+                    dict(lora_rank=16), dict(lora_rank=32, interleave=True)):
+        if options.get("lora_rank") and n % 256:
+            continue  # the rank forms take N in multiples of 256
+        out, want, offsets = _gemm_case(device, counts, n, k, seed=n + k, **options)
+        assert torch.isfinite(out).all(), options
+        assert worst_cell_rel(out, want, offsets.tolist()) < 4e-3, options
+    if n % 256:
+        return
+    g = torch.Generator().manual_seed(n * k)
+    offsets = _ragged(counts).to(device)
+    rows, experts, tokens = int(offsets[-1]), len(counts), 37
+    slots = torch.randint(0, 3 * tokens, (rows,), generator=g).to(torch.int32).to(device)
+    x = torch.randn(tokens, k, generator=g).to(torch.bfloat16).to(device)
+    routed = x[(slots // 3).long()]
+    tq, ts = K.quantize_token_rows(x)
+    xq, xs = K.quantize_rows(routed)
+    w = (torch.randn(experts, n, k, generator=g) * 0.02).to(device)
+    wq, ws = K.quantize_weight_blocks(w)
+    for interleave in (False, True):
+        assert torch.equal(
+            K.gemm_gathered(tq, ts, slots, wq, ws, offsets, interleave=interleave, rows_div=3),
+            K.gemm(xq, xs, wq, ws, offsets, interleave=interleave))
+    kq, ks = K.quantize_weight_blocks(w.transpose(1, 2).contiguous())
+    want = K.gemm(xq, xs, K.transpose_fp8(kq), ks, offsets, transposed_scale=True)
+    assert torch.equal(K.gemm_kmajor(xq, xs, kq, ks, offsets), want)
+    assert torch.equal(K.gemm_gathered(tq, ts, slots, kq, ks, offsets, kmajor=True, rows_div=3),
+                       want)
+    h, act, act_s = K.gemm_swiglu(xq, xs, wq, ws, offsets)
+    assert torch.equal(h, K.gemm(xq, xs, wq, ws, offsets, interleave=True))
+    q_ref, s_ref = K.swiglu_quantize(h)
+    assert torch.equal(_bytes(act), _bytes(q_ref)) and torch.equal(act_s, s_ref)
+    rq, _, rs, _ = K.quantize_weights_current(w)
+    cq, cs = K.quantize_rows_current(routed)
+    out = K.gemm_rowwise(cq, cs, rq, rs, offsets)
+    want = O.rowwise_gemm(cq.cpu(), cs.cpu(), rq.cpu(), rs.cpu(), offsets.cpu())
+    assert worst_cell_rel(out.cpu(), want, offsets.tolist()) < 4e-3
+    ctq, cts = K.quantize_rows_current(x)
+    assert torch.equal(K.gemm_rowwise_gathered(ctq, cts, slots, rq, rs, offsets, rows_div=3), out)
+    z = (torch.randn(rows, 16, generator=g) * 0.5).to(torch.bfloat16)
+    b = (torch.randn(experts, n, 16, generator=g) * 0.1).to(torch.bfloat16)
+    out = K.gemm_rowwise(cq, cs, rq, rs, offsets, lora=(z.to(device), b.to(device)))
+    for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
+        want[lo:hi] += z[lo:hi].double() @ b[e].double().t()
+    assert worst_cell_rel(out.cpu(), want, offsets.tolist()) < 4e-3
+
+
+
 @pytest.mark.parametrize("tokens,top_k,experts,k,n,form", [
     (2000, 4, 16, 512, 512, "up"),           # gate/up interleave, partial row tiles
     (1000, 3, 8, 128, 256, "plain"),         # one K step: the next tile's rows at once
