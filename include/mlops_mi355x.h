@@ -496,6 +496,66 @@ int mi355x_gemm_fp8_block_wgrad(const uint8_t* p, const float* p_scale, int m_fe
                                 int padded, const int32_t* offsets, int experts, void* out,
                                 int out_fp32, void* stream);
 
+/* ------------------------------------------------------------- layer ---- */
+
+/* Launch sequences of one layer pass: the entry points above, in order, from
+ * one call and one workspace (each the same kernels, arguments and results).
+ *
+ * mi355x_moe_route: router_topk, permute_plan and router_stats on the logits
+ * (moe_router.py:235-344; moe_dispatch.py:106-119; moe_common.py:32-71).
+ * mi355x_moe_down: SwiGLU and its quantizer on h13 [A, 2I], the down GEMM
+ * (row_scaled: the per-row forms) and the combine (sonicmoe/moe.py:441-514).
+ * mi355x_moe_block_bwd: the block-FP8 backward from r = dy @ W2 [A, I] to the
+ * input gradient (before the router's share), the weight gradients and the
+ * logit gradient's pieces (sonicmoe/moe.py:346-431). */
+size_t mi355x_moe_route_workspace_size(int tokens, int experts, int top_k, int segments,
+                                       int nchunks);
+int mi355x_moe_route(const float* logits, int tokens, int experts, int top_k, int mode,
+                     const float* bias, int n_group, int topk_group, float routed_scaling,
+                     const int32_t* forced_ids, int segments, const int32_t* seg_offsets,
+                     const int32_t* chunk_table, int nchunks, float* weights, int32_t* ids,
+                     int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
+                     float* aux, float* prob_sum, void* workspace, size_t workspace_bytes,
+                     void* stream);
+size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter);
+int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidden, int inter, float limit,
+                    int row_scaled, const uint8_t* w2, const float* w2_scale, int experts,
+                    const int32_t* offsets, const int32_t* slots, const float* weights,
+                    const void* residual, void* out, void* workspace, size_t workspace_bytes,
+                    void* stream);
+
+typedef struct mi355x_moe_block_bwd_args {
+  const void* r;               /* bf16 [A, I] */
+  const void* h13;             /* bf16 [A, 2I] interleaved */
+  const void* x;               /* bf16 [T, H] */
+  const void* dy;              /* bf16 [T, H] */
+  const float* logits;         /* [T, E] */
+  const float* route_weights;  /* [T, k] */
+  const int32_t* route_ids;    /* [T, k] */
+  const int32_t* order;        /* [A] */
+  const int32_t* offsets;      /* [E + 1] */
+  const int32_t* slots;        /* [T, k] */
+  const uint8_t* w13;          /* [E, 2I, H] (w13_kmajor) or its transpose [E, H, 2I] */
+  const float* w13_scale;      /* [E, 2I/128, H/128] either way */
+  const float* grad_aux;       /* [1] or NULL */
+  const float* grad_prob_sum;  /* [E] or NULL */
+  const int32_t* seg_offsets;  /* as mi355x_router_topk_bwd */
+  const int32_t* seg_counts;
+  void* grad_x;                /* bf16 [T, H] */
+  void* pieces;                /* bf16 [T, 2E] */
+  void* grad_w13;              /* [E, 2I, H] or NULL: not wanted */
+  void* grad_w2;               /* [E, H, I] or NULL */
+  float* grad_router;          /* [E, H] or NULL; widths of mi355x_router_weight_grad */
+  void* workspace;
+  uint64_t workspace_bytes;
+  int32_t tokens, hidden, inter, experts, top_k, mode, segments, w13_kmajor, weight_grads_fp32;
+  float limit;
+} mi355x_moe_block_bwd_args;
+size_t mi355x_moe_block_bwd_workspace_size(int tokens, int hidden, int inter, int experts,
+                                           int top_k, int need_w13, int need_w2,
+                                           int router_kernel);
+int mi355x_moe_block_bwd(const mi355x_moe_block_bwd_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

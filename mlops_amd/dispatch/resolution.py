@@ -1,7 +1,7 @@
 """Choosing an implementation for one call.
 
-Every registered implementation of the operation is asked whether it
-supports the call (metadata only). The selection rule is the reference's
+The registered implementations of the operation are asked whether they
+support the call (metadata only). The selection rule is the reference's
 (``src/mlops/dispatch/resolution.py``): a forced ID is taken if, and only if,
 it supports the call; otherwise the supporting implementation with the
 highest priority, ties going to the lexicographically smaller ID. The
@@ -74,7 +74,19 @@ def explain_implementation(operation: str, *args, surface: str = "semantic",
 
 def resolve_implementation(operation: str, *args, surface: str = "semantic",
                            **kwargs) -> Implementation:
-    """The implementation to run; RuntimeError with every refusal otherwise."""
+    """The implementation to run; RuntimeError with every refusal otherwise.
+
+    Candidates are asked in order of preference and the first that supports
+    the call is the selection :func:`explain_implementation` makes; the others
+    are only asked to explain a refusal."""
+    table = implementations_for(operation)
+    forced = implementation_override(operation)
+    candidates = (sorted(table.values(), key=_preference) if forced is None
+                  else [table[forced]] if forced in table else [])
+    for record in candidates:
+        if _verdict(record, surface, args, kwargs).supported:
+            record_dispatch(str(operation), record.implementation_id)
+            return record
     explanation = explain_implementation(operation, *args, surface=surface, **kwargs)
     if explanation.selected is None:
         refusals = "; ".join(f"{key}: {verdict.reason}"

@@ -12,6 +12,7 @@ Layouts: routed rows ``A = tokens * top_k`` are in expert-sorted order;
 from __future__ import annotations
 
 import ctypes
+import struct
 from typing import Sequence
 
 import torch
@@ -132,7 +133,7 @@ def _ptr(t: torch.Tensor | None):
 
 
 def _stream(device: torch.device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _on_gpu(*tensors: torch.Tensor | None) -> torch.device:
@@ -1001,3 +1002,184 @@ def wgrad(p, p_scale, q, q_scale, offsets, *, out_dtype=torch.bfloat16, rows=Non
         _stream(device),
     )
     return out
+
+
+# ------------------------------------------------------------------- layer
+# Steps that always follow one another in a layer pass, enqueued by one native
+# call (csrc/layer.hip) from one workspace. With a launch timer installed they
+# go through the single-kernel wrappers instead, so that each kernel is timed;
+# the kernels, their arguments and results are the same.
+def route(logits, top_k: int, mode: str, lengths: Sequence[int], *, bias=None, n_group=1,
+          topk_group=1, routed_scaling=1.0, forced_ids=None):
+    """``(weights, ids, counts, offsets, order, slots, aux, prob_sum)``:
+    :func:`router_topk`, :func:`permute_plan` and :func:`router_stats` on fp32
+    ``logits [T, E]`` (``mi355x_moe_route``)."""
+    if _TIMER is not None:
+        weights, ids = router_topk(logits, top_k, mode, bias=bias, n_group=n_group,
+                                   topk_group=topk_group, routed_scaling=routed_scaling,
+                                   forced_ids=forced_ids)
+        counts, offsets, order, slots = permute_plan(ids, logits.shape[1])
+        aux, prob_sum, _, _ = router_stats(logits, ids, top_k, mode, lengths)
+        return weights, ids, counts, offsets, order, slots, aux, prob_sum
+    if mode not in ROUTING_MODES:
+        raise ValueError(f"unsupported routing mode {mode!r}")
+    if logits.dtype != torch.float32 or logits.ndim != 2:
+        raise ValueError("router logits must be fp32 [tokens, experts]")
+    tokens, experts = logits.shape
+    if bias is not None:
+        bias = bias.float().contiguous()
+        if bias.shape != (experts,):
+            raise ValueError("router bias must be [experts]")
+    if forced_ids is not None:
+        forced_ids = forced_ids.to(device=logits.device, dtype=torch.int32).contiguous()
+        _check(forced_ids, (tokens, top_k), torch.int32, "forced_ids")
+    device = _on_gpu(logits, bias, forced_ids)
+    seg_offsets, table, nchunks = segment_tables(lengths, tokens, device)
+    segments = max(1, len(lengths))
+    weights = torch.empty((tokens, top_k), dtype=torch.float32, device=device)
+    ids = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
+    counts = torch.empty(experts, dtype=torch.int64, device=device)
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device=device)
+    order = torch.empty(tokens * top_k, dtype=torch.int32, device=device)
+    slots = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
+    aux = torch.empty((), dtype=torch.float32, device=device)
+    prob_sum = torch.empty(experts, dtype=torch.float32, device=device)
+    size = _native.query("mi355x_moe_route_workspace_size", tokens, experts, top_k, segments,
+                         nchunks)
+    work = torch.empty(size, dtype=torch.uint8, device=device)
+    _native.call("mi355x_moe_route", _ptr(logits), tokens, experts, top_k, ROUTING_MODES[mode],
+                 _ptr(bias), n_group, topk_group, routed_scaling, _ptr(forced_ids), segments,
+                 _ptr(seg_offsets), _ptr(table), nchunks, _ptr(weights), _ptr(ids), _ptr(counts),
+                 _ptr(offsets), _ptr(order), _ptr(slots), _ptr(aux), _ptr(prob_sum), _ptr(work),
+                 size, _stream(device))
+    return weights, ids, counts, offsets, order, slots, aux, prob_sum
+
+
+def moe_down(h13, w2, w2_scale, offsets, slots, weights, residual, limit=None, *,
+             row_scaled=False):
+    """``residual + sum_j weights[t, j] y[slots[t, j]]`` for the down projection
+    ``y`` of ``h13``'s quantized SwiGLU: :func:`swiglu_quantize`, :func:`gemm`
+    and :func:`combine`, or with ``row_scaled`` the per-row forms
+    (``mi355x_moe_down``)."""
+    if _TIMER is not None:
+        if row_scaled:
+            aq, scales = swiglu_quantize_rows_current(h13, limit)
+            y = gemm_rowwise(aq, scales, w2, w2_scale, offsets)
+        else:
+            aq, scales = swiglu_quantize(h13, limit)
+            y = gemm(aq, scales, w2, w2_scale, offsets)
+        return combine(y, slots, weights, residual)
+    tokens, top_k = slots.shape
+    experts, hidden, inter = w2.shape
+    rows = tokens * top_k
+    _check(h13, (rows, 2 * inter), torch.bfloat16, "h13")
+    if w2.dtype != FP8:
+        raise ValueError("moe_down takes an e4m3 weight [E, H, I]")
+    _check(w2_scale, (experts, hidden) if row_scaled else (experts, hidden // 128, inter // 128),
+           torch.float32, "weight scales")
+    _check(offsets, (experts + 1,), torch.int32, "offsets")
+    _check(weights, (tokens, top_k), torch.float32, "route weights")
+    _check(residual, (tokens, hidden), torch.bfloat16, "residual")
+    device = _on_gpu(h13, w2, w2_scale, offsets, slots, weights, residual)
+    out = torch.empty_like(residual)
+    size = _native.query("mi355x_moe_down_workspace_size", rows, hidden, inter)
+    work = torch.empty(size, dtype=torch.uint8, device=device)
+    _native.call("mi355x_moe_down", _ptr(h13), tokens, top_k, hidden, inter, _limit(limit),
+                 int(row_scaled), _ptr(w2), _ptr(w2_scale), experts, _ptr(offsets), _ptr(slots),
+                 _ptr(weights), _ptr(residual), _ptr(out), _ptr(work), size, _stream(device))
+    return out
+
+
+# mi355x_moe_block_bwd_args: 22 pointers, the workspace size, nine ints, a float.
+_BACKWARD_ARGS = struct.Struct("=23Q9if")
+
+
+def router_grad_on_kernel(x, experts: int) -> bool:
+    """Whether ``mi355x_router_weight_grad`` forms the router weight gradient:
+    fewer than 64 experts would leave most of its 128-expert tile idle."""
+    return experts % 8 == 0 and experts >= 64 and x.shape[1] % 256 == 0
+
+
+def moe_block_backward(r, h13, x, dy, logits, route_weights, route_ids, order, offsets, slots,
+                       w13, w13_scale, *, w13_kmajor, mode, grad_aux=None, grad_prob_sum=None,
+                       seg_offsets=None, seg_counts=None, limit=None, need_w13=True,
+                       need_w2=True, need_router=True, weight_grad_dtype=torch.bfloat16):
+    """The block-FP8 backward from ``r = dy @ W2 [A, I]`` on: ``(grad_x bf16
+    [T, H] without the router's share, grad_w13 | None, grad_w2 | None, pieces
+    bf16 [T, 2E], grad_router fp32 [E, H] | None)``. ``w13`` is the weight as
+    stored (``w13_kmajor``) or its transposed copy; ``grad_router`` is formed
+    where :func:`router_grad_on_kernel` says so (``mi355x_moe_block_bwd``)."""
+    tokens, top_k = slots.shape
+    hidden, inter, experts = x.shape[1], r.shape[1], logits.shape[1]
+    rows = tokens * top_k
+    router_kernel = need_router and router_grad_on_kernel(x, experts)
+    if grad_aux is not None:
+        grad_aux = grad_aux.float().reshape(1).contiguous()
+    if grad_prob_sum is not None:
+        grad_prob_sum = grad_prob_sum.float().contiguous()
+    if _TIMER is not None:
+        padded = wgrad_padded_rows(rows, experts)
+        blocks = padded_row_blocks(offsets, padded)
+        dhq, dhs, dh_t, dh_ts, ap_t, ap_ts, dscore, _ = swiglu_bwd_quantize(
+            r, h13, route_weights.reshape(-1), order, offsets, padded=padded, limit=limit,
+            transposed_dh=need_w13, transposed_ap=need_w2, row_blocks=blocks)
+        grad_w13 = grad_w2 = grad_router = None
+        gathered = dict(gather=order, gather_div=top_k, padded=padded, row_blocks=blocks)
+        if need_w2:
+            dy_t, dy_ts, _ = quantize_transpose(dy, offsets, rows, **gathered)
+            grad_w2 = wgrad(dy_t, dy_ts, ap_t, ap_ts, offsets, out_dtype=weight_grad_dtype,
+                            rows=rows)
+        dx = (gemm_kmajor(dhq, dhs, w13, w13_scale, offsets) if w13_kmajor
+              else gemm(dhq, dhs, w13, w13_scale, offsets, transposed_scale=True))
+        if need_w13:
+            x_t, x_ts, _ = quantize_transpose(x, offsets, rows, **gathered)
+            grad_w13 = wgrad(dh_t, dh_ts, x_t, x_ts, offsets, out_dtype=weight_grad_dtype,
+                             rows=rows)
+        grad_x = unpermute_sum(dx, slots)
+        pieces = router_backward(
+            logits, route_weights, route_ids, dscore, slots, mode, grad_aux=grad_aux,
+            grad_prob_sum=grad_prob_sum, offsets=offsets, seg_offsets=seg_offsets,
+            seg_counts=seg_counts, pieces=True)
+        if router_kernel:
+            grad_router = router_weight_grad(pieces, x)
+        return grad_x, grad_w13, grad_w2, pieces, grad_router
+    for name, t, shape, dtype in (
+            ("r", r, (rows, inter), torch.bfloat16),
+            ("h13", h13, (rows, 2 * inter), torch.bfloat16),
+            ("x", x, (tokens, hidden), torch.bfloat16),
+            ("dy", dy, (tokens, hidden), torch.bfloat16),
+            ("logits", logits, (tokens, experts), torch.float32),
+            ("route weights", route_weights, (tokens, top_k), torch.float32),
+            ("route ids", route_ids, (tokens, top_k), torch.int32),
+            ("order", order, (rows,), torch.int32),
+            ("offsets", offsets, (experts + 1,), torch.int32),
+            ("slots", slots, (tokens, top_k), torch.int32),
+            ("w13", w13, (experts, 2 * inter, hidden) if w13_kmajor
+             else (experts, hidden, 2 * inter), FP8),
+            ("w13 scales", w13_scale, (experts, 2 * inter // 128, hidden // 128), torch.float32)):
+        _check(t, shape, dtype, name)
+    device = _on_gpu(r, h13, x, dy, logits, route_weights, route_ids, order, offsets, slots, w13,
+                     w13_scale, grad_aux, grad_prob_sum, seg_offsets, seg_counts)
+    fp32 = weight_grad_dtype == torch.float32
+    grad_x = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=device)
+    pieces = torch.empty((tokens, 2 * experts), dtype=torch.bfloat16, device=device)
+    grad_w13 = grad_w2 = grad_router = None
+    if need_w13:
+        grad_w13 = torch.empty((experts, 2 * inter, hidden), dtype=weight_grad_dtype,
+                               device=device)
+    if need_w2:
+        grad_w2 = torch.empty((experts, hidden, inter), dtype=weight_grad_dtype, device=device)
+    if router_kernel:
+        grad_router = torch.empty((experts, hidden), dtype=torch.float32, device=device)
+    size = _native.query("mi355x_moe_block_bwd_workspace_size", tokens, hidden, inter, experts,
+                         top_k, int(need_w13), int(need_w2), int(router_kernel))
+    work = torch.empty(size, dtype=torch.uint8, device=device)
+    pointers = [0 if t is None else t.data_ptr() for t in (
+        r, h13, x, dy, logits, route_weights, route_ids, order, offsets, slots, w13, w13_scale,
+        grad_aux, grad_prob_sum, seg_offsets, seg_counts, grad_x, pieces, grad_w13, grad_w2,
+        grad_router, work)]
+    _native.call("mi355x_moe_block_bwd", _BACKWARD_ARGS.pack(
+        *pointers, size, tokens, hidden, inter, experts, top_k, ROUTING_MODES[mode],
+        1 if seg_counts is None else seg_counts.shape[0], int(w13_kmajor), int(fp32),
+        _limit(limit)), _stream(device))
+    return grad_x, grad_w13, grad_w2, pieces, grad_router

@@ -165,20 +165,17 @@ def forward_routed(
         logits = router.router_logits(x, router_weight)
         forced = next_override(rows, experts, top_k, x.device) if use_routing_override else None
         bias = None if router_bias is None or router_bias.numel() == 0 else router_bias
-        weights, ids = kernels.router_topk(
-            logits, int(top_k), routing_mode, bias=bias, n_group=int(n_group),
+        weights, ids, counts, offsets, order, slots, aux, probability_sum = kernels.route(
+            logits, int(top_k), routing_mode, lengths, bias=bias, n_group=int(n_group),
             topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced,
         )
-        counts, offsets, order, slots = kernels.permute_plan(ids, experts)
         # GEMM, then the SwiGLU pass: measured faster than the fused epilogue
         # of mi355x_gemm_fp8_block_swiglu, whose activation math runs while
         # every wave of the CU is in the epilogue (no MFMA work to hide it).
         h13 = routed_rows_gemm(x, slots, order, int(top_k), (w13_data, w13_scale), offsets,
                                interleave=True)
-        aq, as_ = kernels.swiglu_quantize(h13, swiglu_limit)
-        y = kernels.gemm(aq, as_, w2_data, w2_scale, offsets)
-        output = kernels.combine(y, slots, weights, base)
-        aux, probability_sum, _, _ = kernels.router_stats(logits, ids, int(top_k), routing_mode, lengths)
+        output = kernels.moe_down(h13, w2_data, w2_scale, offsets, slots, weights, base,
+                                  swiglu_limit)
     return (output.reshape(h2.shape), aux, counts, probability_sum, logits, weights, ids, order,
             offsets, slots, h13)
 
@@ -218,45 +215,71 @@ def backward_routed(
             dy = dy.to(torch.bfloat16)
         # Through the down projection: r = dy_routed @ W2, then SwiGLU backward.
         r = routed_rows_gemm(dy, slots, order, int(top_k), w2, offsets, input_gradient=True)
-        # SwiGLU backward fused with the quantizers of its outputs: dh row-
-        # quantized for the input gradient, dh and a' transposed for the
-        # weight gradients (each only when that gradient is wanted).
-        padded = kernels.wgrad_padded_rows(assignments, experts)
-        blocks = kernels.padded_row_blocks(offsets, padded)
-        dhq, dhs, dh_t, dh_ts, ap_t, ap_ts, dscore, _ = kernels.swiglu_bwd_quantize(
-            r, h13, route_weights.reshape(-1), order, offsets, padded=padded, limit=swiglu_limit,
-            transposed_dh=need_w13, transposed_ap=need_w2, row_blocks=blocks,
+        # Then, in one native sequence: the SwiGLU backward fused with the
+        # quantizers of its outputs (dh row-quantized for the input gradient,
+        # dh and a' transposed for the weight gradients that are wanted), the
+        # two weight gradients, dx = dh @ W13 (gate rows, then up rows) summed
+        # per token, and the logit gradient's bf16 pieces.
+        grad_aux, grad_probability_sum, seg_counts, seg_offsets = _routing_cotangents(
+            grad_aux, grad_probability_sum, logits, route_ids, int(top_k), routing_mode, lengths)
+        w13_operand, w13_kmajor = _input_gradient_operand(w13)
+        grad_h2, grad_w13, grad_w2, pieces, grad_router = kernels.moe_block_backward(
+            r, h13, x, dy, logits, route_weights, route_ids, order, offsets, slots, w13_operand,
+            w13_scale, w13_kmajor=w13_kmajor, mode=routing_mode, grad_aux=grad_aux,
+            grad_prob_sum=grad_probability_sum, seg_offsets=seg_offsets, seg_counts=seg_counts,
+            limit=swiglu_limit, need_w13=need_w13, need_w2=need_w2, need_router=need_router,
+            weight_grad_dtype=direct,
         )
-        if need_w2:
-            dy_t, dy_ts, _ = kernels.quantize_transpose(
-                dy, offsets, assignments, gather=order, gather_div=int(top_k), padded=padded,
-                row_blocks=blocks,
-            )
-            grad_w2 = _grad_at(kernels.wgrad(dy_t, dy_ts, ap_t, ap_ts, offsets, out_dtype=direct,
-                                             rows=assignments),
-                               weight_grad_dtype)
-        else:
-            grad_w2 = skipped_gradient(h2, weight_grad_dtype)
-        # Through the up projection: dx = dh @ W13 (gate rows, then up rows).
-        dx = input_gradient_gemm(dhq, dhs, w13, offsets)
-        if need_w13:
-            x_t, x_ts, _ = kernels.quantize_transpose(
-                x, offsets, assignments, gather=order, gather_div=int(top_k), padded=padded,
-                row_blocks=blocks,
-            )
-            grad_w13 = _grad_at(kernels.wgrad(dh_t, dh_ts, x_t, x_ts, offsets, out_dtype=direct,
-                                              rows=assignments),
-                                weight_grad_dtype)
-        else:
-            grad_w13 = skipped_gradient(h2, weight_grad_dtype)
-        grad_h2 = kernels.unpermute_sum(dx, slots)
-        grad_router = routing_backward(
-            grad_h2, x, router_weight, logits, route_weights, route_ids, dscore, slots, offsets,
-            grad_aux, grad_probability_sum, top_k=top_k, routing_mode=routing_mode,
-            lengths=lengths, router_dtype=router_dtype, need_router=need_router,
-        )
+        grad_w13 = (_grad_at(grad_w13, weight_grad_dtype) if need_w13
+                    else skipped_gradient(h2, weight_grad_dtype))
+        grad_w2 = (_grad_at(grad_w2, weight_grad_dtype) if need_w2
+                   else skipped_gradient(h2, weight_grad_dtype))
+        grad_router = _router_gradients(grad_h2, x, router_weight, pieces, grad_router,
+                                        router_dtype, need_router)
     grad_residual = grad_output.clone() if need_residual else grad_output.new_empty(0)
     return (grad_h2.reshape(h2.shape).to(h2.dtype), grad_residual, grad_router, grad_w13, grad_w2)
+
+
+def _routing_cotangents(grad_aux, grad_probability_sum, logits, route_ids, top_k, routing_mode,
+                        lengths):
+    """``(grad_aux, grad_probability_sum, seg_counts, seg_offsets)`` for the
+    logit gradient: an empty cotangent is None, and the per-sequence aux
+    gradient gets its segments' counts."""
+    if grad_aux is not None and grad_aux.numel() == 0:
+        grad_aux = None
+    if grad_probability_sum is not None and grad_probability_sum.numel() == 0:
+        grad_probability_sum = None
+    seg_offsets = seg_counts = None
+    if routing_mode == "sigmoid_noaux_tc" and grad_aux is not None:
+        _, _, seg_counts, seg_offsets = kernels.router_stats(
+            logits, route_ids, top_k, routing_mode, lengths
+        )
+    return grad_aux, grad_probability_sum, seg_counts, seg_offsets
+
+
+def _aligned(gradient, like):
+    """``gradient`` with ``like``'s strides."""
+    if gradient.stride() == like.stride():
+        return gradient
+    aligned = torch.empty_strided(gradient.shape, like.stride(), dtype=gradient.dtype,
+                                  device=gradient.device)
+    return aligned.copy_(gradient)
+
+
+def _router_gradients(grad_h2, x, router_weight, pieces, formed, router_dtype, need_router):
+    """The router weight's gradient from the logit gradient's bf16 pieces
+    (``formed``: the fp32 gradient where a kernel has formed it already; a
+    placeholder when not needed); the router's input gradient is added to
+    ``grad_h2`` in place."""
+    if not need_router:
+        gradient = skipped_gradient(router_weight, router_dtype)
+    elif formed is not None:
+        gradient = _aligned(formed.to(router_dtype), router_weight)
+    else:
+        gradient = _aligned(
+            router.router_weight_gradient_from_pieces(pieces, x, router_dtype), router_weight)
+    router.add_router_input_gradient_from_pieces_(grad_h2, pieces, router_weight)
+    return gradient
 
 
 def routing_backward(grad_h2, x, router_weight, logits, route_weights, route_ids, dscore, slots,
@@ -267,15 +290,8 @@ def routing_backward(grad_h2, x, router_weight, logits, route_weights, route_ids
     placeholder when not needed) and adds the router's input gradient to
     ``grad_h2`` in place. An empty ``grad_aux`` / ``grad_probability_sum``
     stands for a zero cotangent."""
-    if grad_aux is not None and grad_aux.numel() == 0:
-        grad_aux = None
-    if grad_probability_sum is not None and grad_probability_sum.numel() == 0:
-        grad_probability_sum = None
-    seg_offsets = seg_counts = None
-    if routing_mode == "sigmoid_noaux_tc" and grad_aux is not None:
-        _, _, seg_counts, seg_offsets = kernels.router_stats(
-            logits, route_ids, int(top_k), routing_mode, lengths
-        )
+    grad_aux, grad_probability_sum, seg_counts, seg_offsets = _routing_cotangents(
+        grad_aux, grad_probability_sum, logits, route_ids, int(top_k), routing_mode, lengths)
     # bf16 activations: the kernel writes the cotangent's bf16 pieces, the
     # operands of both router GEMMs, in place of fp32 logit gradients.
     split = (router.operand_dtype(x) == torch.bfloat16 and grad_h2.dtype == torch.bfloat16
@@ -286,24 +302,11 @@ def routing_backward(grad_h2, x, router_weight, logits, route_weights, route_ids
         seg_offsets=seg_offsets, seg_counts=seg_counts, pieces=split,
     )
     if split:
-        if need_router:
-            grad_router = router.router_weight_gradient_from_pieces(grad_logits, x, router_dtype)
-            if grad_router.stride() != router_weight.stride():
-                aligned = torch.empty_strided(grad_router.shape, router_weight.stride(),
-                                              dtype=grad_router.dtype, device=grad_router.device)
-                aligned.copy_(grad_router)
-                grad_router = aligned
-        else:
-            grad_router = skipped_gradient(router_weight, router_dtype)
-        router.add_router_input_gradient_from_pieces_(grad_h2, grad_logits, router_weight)
-        return grad_router
+        return _router_gradients(grad_h2, x, router_weight, grad_logits, None, router_dtype,
+                                 need_router)
     if need_router:
-        grad_router = router.router_weight_gradient(grad_logits, x, router_dtype)
-        if grad_router.stride() != router_weight.stride():
-            aligned = torch.empty_strided(grad_router.shape, router_weight.stride(),
-                                          dtype=grad_router.dtype, device=grad_router.device)
-            aligned.copy_(grad_router)
-            grad_router = aligned
+        grad_router = _aligned(router.router_weight_gradient(grad_logits, x, router_dtype),
+                               router_weight)
     else:
         grad_router = skipped_gradient(router_weight, router_dtype)
     router.add_router_input_gradient_(grad_h2, grad_logits, router_weight)
@@ -368,13 +371,20 @@ def input_gradient_gemm(aq, a_scale, weight, offsets):
     scale[, data_t])``): through a transposed copy the weight carries, else
     on the data as stored (``mi355x_gemm_fp8_block_kmajor``, bitwise the
     same), else (N not a multiple of 256) through a copy transposed now."""
-    data, scale = weight[0], weight[1]
+    operand, kmajor = _input_gradient_operand(weight)
+    if kmajor:
+        return kernels.gemm_kmajor(aq, a_scale, operand, weight[1], offsets)
+    return kernels.gemm(aq, a_scale, operand, weight[1], offsets, transposed_scale=True)
+
+
+def _input_gradient_operand(weight):
+    """``(operand, kmajor)`` of :func:`input_gradient_gemm`: the transposed
+    copy, or the data as stored."""
     if len(weight) == 3:
-        return kernels.gemm(aq, a_scale, weight[2], scale, offsets, transposed_scale=True)
-    if data.shape[2] % 256 == 0:
-        return kernels.gemm_kmajor(aq, a_scale, data, scale, offsets)
-    return kernels.gemm(aq, a_scale, kernels.transpose_fp8(data), scale, offsets,
-                        transposed_scale=True)
+        return weight[2], False
+    if weight[0].shape[2] % 256 == 0:
+        return weight[0], True
+    return kernels.transpose_fp8(weight[0]), False
 
 
 def available_transposed(container) -> torch.Tensor | None:

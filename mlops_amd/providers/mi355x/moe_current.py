@@ -105,17 +105,13 @@ def forward_routed(h2, residual, router_weight, w13, w2, *, top_k, routing_mode,
         logits = router.router_logits(x, router_weight)
         forced = next_override(rows, experts, top_k, x.device)
         bias = None if router_bias is None or router_bias.numel() == 0 else router_bias
-        weights, ids = kernels.router_topk(
-            logits, int(top_k), routing_mode, bias=bias, n_group=int(n_group),
+        weights, ids, counts, offsets, order, slots, aux, probability_sum = kernels.route(
+            logits, int(top_k), routing_mode, lengths, bias=bias, n_group=int(n_group),
             topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced,
         )
-        counts, offsets, order, slots = kernels.permute_plan(ids, experts)
         h13 = _routed_rows_gemm(x, slots, order, int(top_k), w13[0], w13[2], offsets)
-        aq, as_ = kernels.swiglu_quantize_rows_current(h13, swiglu_limit)
-        y = kernels.gemm_rowwise(aq, as_, w2[0], w2[2], offsets)
-        output = kernels.combine(y, slots, weights, base)
-        aux, probability_sum, _, _ = kernels.router_stats(logits, ids, int(top_k), routing_mode,
-                                                          lengths)
+        output = kernels.moe_down(h13, w2[0], w2[2], offsets, slots, weights, base, swiglu_limit,
+                                  row_scaled=True)
     return (output.reshape(h2.shape), aux, counts, probability_sum, logits, weights, ids, order,
             offsets, slots, h13)
 

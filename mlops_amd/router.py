@@ -75,11 +75,11 @@ def router_weight_gradient_from_pieces(pieces, hidden, dtype) -> torch.Tensor:
     hipBLASLt."""
     experts = pieces.shape[1] // 2
     hidden = hidden.reshape(-1, hidden.shape[-1])
-    if (pieces.is_cuda and hidden.dtype == torch.bfloat16 and experts % 8 == 0
-            and experts >= 64 and hidden.shape[1] % 256 == 0):
+    if pieces.is_cuda and hidden.dtype == torch.bfloat16:
         from . import kernels
 
-        return kernels.router_weight_grad(pieces, hidden).to(dtype)
+        if kernels.router_grad_on_kernel(hidden, experts):
+            return kernels.router_weight_grad(pieces, hidden).to(dtype)
     both = split_k_product(pieces, hidden)
     return both[:experts].add_(both[experts:]).to(dtype)
 

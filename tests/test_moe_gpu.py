@@ -545,3 +545,36 @@ def test_gathered_token_rows_equal_permuted_copy_in_the_layer(device, monkeypatc
     names = ["out", "aux", "counts", "psum", "x", "router", "w13", "w2"]
     for name, a, b in zip(names, gathered, permuted, strict=True):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("precision,tokens,experts,top_k,inter,mode", [
+    ("fp8_block", 1, 8, 2, 256, "topk_then_softmax"),        # the smallest call
+    ("fp8_block", 97, 64, 8, 256, "softmax_then_topk"),      # router gradient on its kernel
+    ("fp8_block", 130, 8, 3, 384, "sigmoid_noaux_tc"),       # w2's transposed copy, sequences
+    ("fp8_current", 65, 16, 4, 256, "topk_then_softmax"),
+])
+def test_launch_sequences_equal_single_kernel_calls(device, precision, tokens, experts, top_k,
+                                                    inter, mode):
+    """The layer's native launch sequences give the bytes of the same kernels
+    called one at a time (as they are while a launch timer is installed)."""
+    x, res, wr, w13, w2, dy = _inputs(device, tokens=tokens, hidden=256, experts=experts,
+                                      inter=inter, seed=13)
+    lengths = (tokens // 2, tokens - tokens // 2) if mode == "sigmoid_noaux_tc" else None
+
+    def run():
+        leaves = [t.clone().requires_grad_(True) for t in (x, wr, w13, w2)]
+        out, aux, counts, psum = mlops_amd.moe(
+            leaves[0], res, *leaves[1:], top_k=top_k, routing_mode=mode, lengths=lengths,
+            compute_precision=precision, swiglu_limit=2.0)
+        grads = torch.autograd.grad([out, aux, psum], leaves,
+                                    [dy, torch.ones_like(aux) * 0.1, torch.ones_like(psum)])
+        return [out, aux, counts, psum, *grads]
+
+    together = run()
+    K.set_launch_timer(K.LaunchTimer())
+    try:
+        single = run()
+    finally:
+        K.set_launch_timer(None)
+    for a, b in zip(together, single, strict=True):
+        assert torch.equal(a, b)
