@@ -1,11 +1,10 @@
-// Grouped weight-gradient GEMM, pipelined form (both feature counts
-// multiples of 256):
+// Grouped weight-gradient GEMM:
 //   out[e][m][n] = sum over expert e's padded rows k of P[m][k] * Q[n][k]
 // with P, Q the feature-major e4m3 operands written by the transposing
 // quantizer and one power-of-two descale per (feature, 128-row block).
 //
-// Same main loop as the grouped GEMM (gemm_pipe.h: 256 x 256 tile, 8 waves,
-// direct-to-LDS loads, two stages) with one difference: both operands carry
+// wgrad_v2_kernel has the main loop of the grouped GEMM (gemm_pipe.h: 256 x 256
+// tile, 8 waves, direct-to-LDS loads, two stages) with one difference: both operands carry
 // per-row scales that are powers of two, so the MFMA applies them itself
 // (v_mfma_scale_f32_16x16x128_f8f6f4 with E8M0 scales = the fp32 exponent
 // byte) and accumulates across K blocks in place: no VALU work in the loop.
@@ -21,12 +20,16 @@ namespace {
 
 constexpr int kMaxExperts = 512;
 
-// q feature behind B-tile row tr: MFMA column c of block jb feeds output
-// column c * 8 + jb of the wave's 128, so a lane's eight accumulator blocks
-// are eight consecutive output columns.
+// q feature behind B-tile row tr, of MFMA column c of block jb: output column
+// c * 8 + jb of the wave's 128, so that a lane's eight accumulator blocks are
+// eight consecutive bf16 columns (one 16-byte store); with fp32 outputs
+// columns 4c .. 4c + 3 of either half, so that each of the two 16-byte
+// stores of a row fills whole lines (32 bytes per lane, stored as two halves
+// of a line, took 930 us for 1.6 GB of gradients where this takes 271).
+template <bool kFp32>
 __device__ __forceinline__ int feature_col(int tr, int nt) {
-  const int part = tr >> 7, local = tr & 127;
-  return nt * BN + part * 128 + (local & 15) * 8 + (local >> 4);
+  const int part = tr >> 7, local = tr & 127, c = local & 15, jb = local >> 4;
+  return nt * BN + part * 128 + (kFp32 ? (jb >> 2) * 64 + c * 4 + (jb & 3) : c * 8 + jb);
 }
 
 __device__ __forceinline__ int e8m0(float pow2_scale) { return __float_as_int(pow2_scale) >> 23; }
@@ -55,10 +58,11 @@ __device__ __forceinline__ WTile wdescribe(const int* prefix, int per_e, int n_t
   return t;
 }
 
+template <bool kFp32>
 __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
     const uint8_t* __restrict__ p, const float* __restrict__ p_scale, int Mf,
     const uint8_t* __restrict__ q, const float* __restrict__ q_scale, int Nf, int padded,
-    const int32_t* __restrict__ offsets, int experts, void* __restrict__ out, int out_fp32) {
+    const int32_t* __restrict__ offsets, int experts, void* __restrict__ out) {
   __shared__ __align__(1024) uint8_t smem[kStages * STAGE_BYTES];
   __shared__ int prefix[kMaxExperts + 1];
   __shared__ int tmp[kThreads];
@@ -85,7 +89,7 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
 #pragma unroll
     for (int i = 0; i < B_LOADS; ++i) {
       const int tr = (wave * B_LOADS + i) * 8 + (lane >> 3);
-      const uint32_t off = (uint32_t)feature_col(tr, t.nt) * (uint32_t)padded + 16 * ((lane & 7) ^ swz(tr));
+      const uint32_t off = (uint32_t)feature_col<kFp32>(tr, t.nt) * (uint32_t)padded + 16 * ((lane & 7) ^ swz(tr));
       dma16(bbase, off, base + A_BYTES + (wave * B_LOADS + i) * 1024);
     }
     // Scales of this K block, stored in lane order: LDS slot wm*64 + c*4 + i
@@ -101,7 +105,7 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
     } else {
       const int slot = (wave - 4) * 64 + lane;
       const int tr = (slot & ~127) + (slot & 7) * 16 + ((slot >> 3) & 15);
-      dma4(q_scale + kblock * Nf, 4u * (uint32_t)feature_col(tr, t.nt),
+      dma4(q_scale + kblock * Nf, 4u * (uint32_t)feature_col<kFp32>(tr, t.nt),
            sbase + SA_BYTES + (wave - 4) * 256);
     }
   };
@@ -200,19 +204,19 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
       stage ^= 1;
     }
 
-    // Epilogue from registers: lane (row, 8 consecutive columns).
+    // Epilogue from registers: lane (row, its 8 columns; see feature_col).
     const size_t row0 = (size_t)ct.e * Mf + ct.mt * BM + wm * 64;
-    const size_t col0 = (size_t)ct.nt * BN + wn * 128 + (lane & 15) * 8;
+    const size_t col0 = (size_t)ct.nt * BN + wn * 128 + (lane & 15) * (kFp32 ? 4 : 8);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int lrow = i * 16 + 4 * (lane >> 4) + r;
         const size_t off = (row0 + lrow) * Nf + col0;
-        if (out_fp32) {
+        if constexpr (kFp32) {
           float* o = (float*)out + off;
           store_stream(o, make_uint4(__float_as_uint(acc[i][0][r]), __float_as_uint(acc[i][1][r]), __float_as_uint(acc[i][2][r]), __float_as_uint(acc[i][3][r])));
-          store_stream(o + 4, make_uint4(__float_as_uint(acc[i][4][r]), __float_as_uint(acc[i][5][r]), __float_as_uint(acc[i][6][r]), __float_as_uint(acc[i][7][r])));
+          store_stream(o + 64, make_uint4(__float_as_uint(acc[i][4][r]), __float_as_uint(acc[i][5][r]), __float_as_uint(acc[i][6][r]), __float_as_uint(acc[i][7][r])));
         } else {
           uint4 o;
           o.x = pack_bf16x2(acc[i][0][r], acc[i][1][r]);
@@ -229,24 +233,219 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// 128 x 128 tiles, two workgroups per CU: feature counts that are odd
+// multiples of 128, and groups of few rows, where a tile is one or two K
+// steps and its output decides (a 256 x 256 tile's epilogue then runs alone
+// on its CU; two workgroups overlap one's stores with the other's copies).
+// 8 waves in a 4 x 2 grid, wave tile 32 x 64 (2 x 4 blocks), two stages.
+namespace small {
+constexpr int TM = 128, TN = 128;
+constexpr int MB = 2, NB = 4;
+constexpr int A_SIZE = TM * BK, B_SIZE = TN * BK;
+constexpr int STAGE = A_SIZE + B_SIZE + 4 * (TM + TN);
+constexpr int kStores = MB * 4;  // store instructions of a wave's epilogue
+}  // namespace small
+
+template <bool kFp32>
+__global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
+    const uint8_t* __restrict__ p, const float* __restrict__ p_scale, int Mf,
+    const uint8_t* __restrict__ q, const float* __restrict__ q_scale, int Nf, int padded,
+    const int32_t* __restrict__ offsets, int experts, void* __restrict__ out) {
+  using namespace small;
+  __shared__ __align__(1024) uint8_t smem[2 * STAGE];
+  __shared__ int prefix[kMaxExperts + 1];
+  padded_block_prefix<kThreads>(offsets, experts, prefix, (int*)smem);
+  const int n_tiles = Nf / TN;
+  const int per_e = (Mf / TM) * n_tiles;
+  const int total = experts * per_e;
+  const int tid = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lrow = lane >> 3, unit = (lane & 7) ^ (lane >> 3), c = lane & 15;
+
+  struct Tile {
+    int e, mt, nt, k0, nk;
+  };
+  auto describe = [&](int tile) -> Tile {
+    Tile t;
+    t.e = tile / per_e;
+    const int rem = tile - t.e * per_e;
+    t.mt = rem / n_tiles;
+    t.nt = rem - t.mt * n_tiles;
+    t.k0 = __builtin_amdgcn_readfirstlane(prefix[t.e]);
+    t.nk = __builtin_amdgcn_readfirstlane(prefix[t.e + 1]) - t.k0;
+    return t;
+  };
+  // K block kb of tile t into a stage. The Q row behind tile row (jb, c) of a
+  // wave column is feature 4c + jb of its 64, so a lane's four blocks are
+  // four consecutive output columns. Scales in lane order: P's slot
+  // wm * 32 + 2c + i holds row wm * 32 + 16i + c; Q's order is natural.
+  auto issue = [&](const Tile& t, int kb, int stage) {
+    uint8_t* base = smem + stage * STAGE;
+    const size_t block = (size_t)(t.k0 + kb);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int tr = (wave * 2 + i) * 8;
+      dma16(p + (size_t)(t.mt * TM + tr) * padded + block * 128,
+            (uint32_t)lrow * (uint32_t)padded + 16 * unit, base + tr * 128);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int tr = (wave * 2 + i) * 8;
+      const int feature = t.nt * TN + (tr >> 6) * 64 + (tr & 8) * 4 + ((tr >> 4) & 3);
+      dma16(q + (size_t)feature * padded + block * 128,
+            (uint32_t)(4 * lrow) * (uint32_t)padded + 16 * unit, base + A_SIZE + tr * 128);
+    }
+    uint8_t* scales = base + A_SIZE + B_SIZE;
+    if (wave < 2) {
+      const int slot = wave * 64 + lane;
+      const int row = (slot & ~31) + (slot & 1) * 16 + ((slot >> 1) & 15);
+      dma4(p_scale + block * Mf + t.mt * TM, 4u * (uint32_t)row, scales + wave * 256);
+    } else if (wave < 4) {
+      dma4(q_scale + block * Nf + t.nt * TN + (wave - 2) * 64, 4u * (uint32_t)lane,
+           scales + TM * 4 + (wave - 2) * 256);
+    }
+  };
+
+  // XCD-affine ranges balanced by cost, as in wgrad_v2_kernel, with two steps
+  // added to every tile for its output.
+  constexpr int kTileCost = 2;
+  const bool affine = (gridDim.x & 7) == 0;
+  const int xcd = blockIdx.x & 7, cu = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
+  auto range_start = [&](int x) -> int {
+    if (x <= 0) return 0;
+    if (x >= 8) return total;
+    auto before = [&](int e) -> long long {
+      return (long long)per_e * (prefix[e] + kTileCost * e);
+    };
+    const long long bound = before(experts) * x / 8;
+    int lo = 0, hi = experts - 1;  // last e with cost before it <= bound
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (before(mid) <= bound) lo = mid; else hi = mid - 1;
+    }
+    const int cost = prefix[lo + 1] - prefix[lo] + kTileCost;
+    const long long j = (bound - before(lo) + cost - 1) / cost;
+    return lo * per_e + (int)(j < per_e ? j : per_e);
+  };
+  const int first = __builtin_amdgcn_readfirstlane(affine ? range_start(xcd) : 0);
+  const int last = __builtin_amdgcn_readfirstlane(affine ? range_start(xcd + 1) : total);
+  auto tile_at = [&](int r) -> int {
+    const int t = affine ? first + r * per_xcd + cu : tile_of(r, blockIdx.x, gridDim.x);
+    return t < last ? t : -1;
+  };
+  // The issue pointer runs one step ahead, over the tiles that have steps.
+  int i_round = 0, i_step = 0, i_slot = 0;
+  int i_tile = tile_at(0);
+  if (i_tile < 0) return;
+  Tile it = describe(i_tile);
+  auto skip_empty = [&]() {
+    while (i_tile >= 0 && it.nk == 0) {
+      i_tile = tile_at(++i_round);
+      if (i_tile >= 0) it = describe(i_tile);
+    }
+  };
+  skip_empty();
+  auto issue_next = [&]() {
+    if (i_tile < 0) return;
+    issue(it, i_step, i_slot);
+    i_slot ^= 1;
+    if (++i_step == it.nk) {
+      i_step = 0;
+      i_tile = tile_at(++i_round);
+      if (i_tile >= 0) it = describe(i_tile);
+      skip_empty();
+    }
+  };
+  issue_next();
+
+  int slot = 0;
+  bool stored = false;  // an epilogue since the last copies were issued
+  for (int round = 0;; ++round) {
+    const int tile = tile_at(round);
+    if (tile < 0) break;
+    const Tile ct = describe(tile);
+    v4f acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int kb = 0; kb < ct.nk; ++kb) {
+      // The copies of this step are older than the last epilogue's stores,
+      // which stay in flight.
+      if (stored)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kStores) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      stored = false;
+      issue_next();
+      const uint8_t* ta = smem + slot * STAGE;
+      const uint8_t* tb = ta + A_SIZE;
+      const float* sa = (const float*)(tb + B_SIZE);
+      const float2 sa2 = *(const float2*)&sa[wm * 32 + c * 2];
+      const float4 sb4 = *(const float4*)&sa[TM + wn * 64 + c * 4];
+      slot ^= 1;
+      v8i af[MB], bf[NB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) af[i] = frag(ta, (wm * MB + i) * 16 + c, lane);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) bf[j] = frag(tb, (wn * NB + j) * 16 + c, lane);
+      const int ea[MB] = {e8m0(sa2.x), e8m0(sa2.y)};
+      const int eb[NB] = {e8m0(sb4.x), e8m0(sb4.y), e8m0(sb4.z), e8m0(sb4.w)};
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) acc[i][j] = mfma_e8(af[i], bf[j], acc[i][j], ea[i], eb[j]);
+    }
+    const size_t row0 = (size_t)ct.e * Mf + ct.mt * TM + wm * 32;
+    const size_t col0 = (size_t)ct.nt * TN + wn * 64 + c * 4;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const size_t at = (row0 + i * 16 + 4 * (lane >> 4) + r) * Nf + col0;
+        if constexpr (kFp32) {
+          store_stream((float*)out + at,
+                       make_uint4(__float_as_uint(acc[i][0][r]), __float_as_uint(acc[i][1][r]),
+                                  __float_as_uint(acc[i][2][r]), __float_as_uint(acc[i][3][r])));
+        } else {
+          store_stream8((uint16_t*)out + at, make_uint2(pack_bf16x2(acc[i][0][r], acc[i][1][r]),
+                                                        pack_bf16x2(acc[i][2][r], acc[i][3][r])));
+        }
+      }
+    }
+    stored = true;
+  }
+}
+
 }  // namespace
 
-// Launches the pipelined kernel; returns 1 if the shape is not its form
-// (feature counts not multiples of 256, or operands beyond 32-bit offsets),
-// in which case the caller uses the general kernel.
-int mi355x_wgrad_v2_launch(const uint8_t* p, const float* p_scale, int m_features,
-                           const uint8_t* q, const float* q_scale, int n_features, int padded,
-                           const int32_t* offsets, int experts, void* out, int out_fp32,
-                           void* stream) {
-  if (m_features % BM != 0 || n_features % BN != 0 || experts > kMaxExperts) return 1;
-  if ((uint64_t)m_features * (uint64_t)padded >= (1ull << 32) ||
-      (uint64_t)n_features * (uint64_t)padded >= (1ull << 32))
-    return 1;
-  const int total = experts * (m_features / BM) * (n_features / BN);
-  const int grid = total < cu_count() ? total : cu_count();
-  hipLaunchKernelGGL(wgrad_v2_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, p,
-                     p_scale, m_features, q, q_scale, n_features, padded, offsets, experts, out,
-                     out_fp32);
+// 256 x 256 tiles where both feature counts are multiples of 256 and the tiles
+// fill the CUs at least once, else 128 x 128 tiles. Measured on MI355X (256-
+// / 128-sided tiles, bf16 out, us): 2048 x 1536, 128 experts 135 / 144 at 1021
+// tokens (0.8 GB written, 5.9 TB/s) and 486 / 654 at 16384; 2048 x 512, 8
+// experts (128 and 512 tiles) 22 / 15 at 2048 tokens and 60 / 37 at 8192.
+// The 128 x 128 kernel it replaces at other widths, with register-staged
+// copies and a VALU fold of the scales, took 271 us for the two gradients of
+// 1152 x 1280 and 640, 16 experts, 12004 rows in fp32; this one takes 62.
+int mi355x_wgrad_launch(const uint8_t* p, const float* p_scale, int m_features, const uint8_t* q,
+                        const float* q_scale, int n_features, int padded, const int32_t* offsets,
+                        int experts, void* out, int out_fp32, void* stream) {
+  bool wide = m_features % BM == 0 && n_features % BN == 0 &&
+              (uint64_t)m_features * (uint64_t)padded < (1ull << 32) &&
+              (uint64_t)n_features * (uint64_t)padded < (1ull << 32);
+  wide = wide && (long long)experts * (m_features / BM) * (n_features / BN) >= cu_count();
+  MI355X_REQUIRE(wide || (uint64_t)padded < (1ull << 27), "wgrad: padded rows beyond 2^27");
+  const int side = wide ? BM : small::TM, slots = wide ? cu_count() : 2 * cu_count();
+  const long long total = (long long)experts * (m_features / side) * (n_features / side);
+  const int grid = total < slots ? (int)total : slots;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, p, p_scale,
+                       m_features, q, q_scale, n_features, padded, offsets, experts, out);
+  };
+  if (wide) out_fp32 ? launch(wgrad_v2_kernel<true>) : launch(wgrad_v2_kernel<false>);
+  else out_fp32 ? launch(wgrad_tile_kernel<true>) : launch(wgrad_tile_kernel<false>);
   MI355X_LAUNCH_CHECK();
-  return 0;
+  return MI355X_OK;
 }

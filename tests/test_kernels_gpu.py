@@ -668,6 +668,38 @@ def test_wgrad_matches_fp64(device, out_dtype, features):
         assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
 
 
+@pytest.mark.parametrize("counts,features", [
+    ([0, 1, 128, 129, 0], (128, 384)),                 # 128 x 128 tiles, odd multiples of 128
+    ([40, 300, 0, 257], (384, 640)),                   # several K blocks, an empty expert
+    ([3] * 31 + [0], (1024, 512)),                     # 256 tiles of 256 x 256: the wide kernel
+    ([130] * 7 + [0] * 18 + [1] * 7, (512, 1024)),
+])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_wgrad_at_both_tile_sizes(device, out_dtype, counts, features):
+    """Both tile sizes and output types against the fp64 sums. fp32: the matrix
+    core aligns the 128 products of one instruction to the largest before it
+    adds them, dropping bits below about 2^-22 of it: 128 such losses against a
+    sum of about sqrt(128) products are at most 128 / sqrt(128) 2^-22 = 3e-6
+    per unit of the largest product over the typical one, which is up to 20
+    for normal operands, 6e-5 of a cell (1e-4 in the test above); bf16: one
+    rounding, 2^-9 of each element (4e-3 of a cell, twice the worst)."""
+    g = torch.Generator().manual_seed(sum(counts))
+    offsets = _ragged(counts)
+    rows = int(offsets[-1])
+    p_rows = torch.randn(rows, features[0], generator=g).to(torch.bfloat16)
+    q_rows = torch.randn(rows, features[1], generator=g).to(torch.bfloat16)
+    pt, pts, padded = K.quantize_transpose(p_rows.to(device), offsets.to(device), rows)
+    qt, qts, _ = K.quantize_transpose(q_rows.to(device), offsets.to(device), rows, padded=padded)
+    out = K.wgrad(pt, pts, qt, qts, offsets.to(device), out_dtype=out_dtype).cpu()
+    want = O.wgrad(pt.cpu(), pts.cpu(), qt.cpu(), qts.cpu(), offsets)
+    tol = 6e-5 if out_dtype == torch.float32 else 4e-3
+    for e, n in enumerate(counts):
+        if n == 0:
+            assert torch.all(out[e] == 0)
+            continue
+        assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
+
+
 def test_combine_and_token_sum(device):
     g = torch.Generator().manual_seed(20)
     tokens, top_k, width, experts = 300, 3, 768, 8
