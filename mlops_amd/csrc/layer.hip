@@ -7,6 +7,13 @@
 // each instead of one per kernel.
 #include "common.h"
 
+// router.hip: the routing of at most 64 tokens; returns 1 outside its range.
+int mi355x_route_small(const float* logits, int tokens, int experts, int top_k, int mode,
+                       const float* bias, int n_group, int topk_group, float routed_scaling,
+                       const int32_t* forced_ids, int segments, float* weights, int32_t* ids,
+                       int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
+                       float* aux, float* prob_sum, void* stream);
+
 namespace {
 
 // Walks a workspace in 256-byte steps; with a null base it only counts.
@@ -120,6 +127,10 @@ extern "C" int mi355x_moe_route(const float* logits, int tokens, int experts, in
   MI355X_REQUIRE(tokens >= 0 && experts > 0 && top_k > 0, "moe_route: bad sizes");
   const RouteSpace s = route_space(workspace, tokens, experts, top_k, segments, nchunks);
   MI355X_REQUIRE(workspace_bytes >= s.total, "moe_route: workspace too small");
+  const int small = mi355x_route_small(logits, tokens, experts, top_k, mode, bias, n_group,
+                                       topk_group, routed_scaling, forced_ids, segments, weights,
+                                       ids, counts, offsets, order, slots, aux, prob_sum, stream);
+  if (small <= 0) return small;
   STEP(mi355x_router_topk(logits, tokens, experts, top_k, mode, bias, n_group, topk_group,
                           routed_scaling, forced_ids, weights, ids, stream));
   STEP(mi355x_permute_plan(ids, tokens * top_k, experts, counts, offsets, order, slots, s.plan,

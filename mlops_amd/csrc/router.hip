@@ -92,15 +92,15 @@ struct LaneBest {
   }
 };
 
+// Top-k of one token by its W-lane group: lane j < top_k gets choice j's id and
+// route weight. `sv`: LDS of the token's wavefront for group-limited selection
+// (W = 64 only).
 template <int W, int PL>
-__global__ void __launch_bounds__(256) router_topk_kernel(
-    const float* __restrict__ logits, int tokens, int experts, int top_k, int mode,
+__device__ __forceinline__ void topk_token(
+    const float* __restrict__ logits, int token, int experts, int top_k, int mode,
     const float* __restrict__ bias, int n_group, int topk_group, float routed_scaling,
-    const int32_t* __restrict__ forced, float* __restrict__ weights, int32_t* __restrict__ ids) {
-  __shared__ float lds_sel[W == 64 ? 4 : 1][W == 64 ? 512 : 1];
+    const int32_t* __restrict__ forced, float* sv, float& weight, int& id) {
   const int lane = threadIdx.x & (W - 1), gbase = lane_id() & ~(W - 1);
-  const int token = blockIdx.x * (256 / W) + threadIdx.x / W;
-  if (token >= tokens) return;
   constexpr int per_lane = PL;  // slots per lane (experts <= W * PL)
   const float* row = logits + (size_t)token * experts;
 
@@ -149,7 +149,6 @@ __global__ void __launch_bounds__(256) router_topk_kernel(
         if (topk_group < n_group) {
           // Group-limited selection: a group's score is the sum of its two
           // largest selection values; keep the topk_group best groups.
-          float* sv = lds_sel[threadIdx.x >> 6];
           SLOTS(i) {
             int e = lane + 64 * i;
             if (e < experts) sv[e] = val[i];
@@ -241,10 +240,53 @@ __global__ void __launch_bounds__(256) router_topk_kernel(
     float s = group_sum<W>(active ? mine : 0.0f);
     w = mine / s * routed_scaling;
   }
-  if (active) {
+  weight = w;
+  id = my_id;
+}
+
+template <int W, int PL>
+__global__ void __launch_bounds__(256) router_topk_kernel(
+    const float* __restrict__ logits, int tokens, int experts, int top_k, int mode,
+    const float* __restrict__ bias, int n_group, int topk_group, float routed_scaling,
+    const int32_t* __restrict__ forced, float* __restrict__ weights, int32_t* __restrict__ ids) {
+  __shared__ float lds_sel[W == 64 ? 4 : 1][W == 64 ? 512 : 1];
+  const int lane = threadIdx.x & (W - 1);
+  const int token = blockIdx.x * (256 / W) + threadIdx.x / W;
+  if (token >= tokens) return;
+  float w;
+  int id;
+  topk_token<W, PL>(logits, token, experts, top_k, mode, bias, n_group, topk_group,
+                    routed_scaling, forced, lds_sel[W == 64 ? threadIdx.x >> 6 : 0], w, id);
+  if (lane < top_k) {
     weights[(size_t)token * top_k + lane] = w;
-    ids[(size_t)token * top_k + lane] = my_id;
+    ids[(size_t)token * top_k + lane] = id;
   }
+}
+
+// A token's logits in a W-lane group -> its routing probabilities (softmax, or
+// the sigmoid scores over their sum), in place.
+template <int W, int PL>
+__device__ __forceinline__ void token_probabilities(float* l, int experts, int mode) {
+  const int lane = threadIdx.x & (W - 1);
+  constexpr int per_lane = PL;
+  float s = 0.0f;
+  if (mode == MI355X_ROUTE_SIGMOID_NOAUX_TC) {
+    SLOTS(i) {
+      int e = lane + W * i;
+      l[i] = e < experts ? sigmoid_f(l[i]) : 0.0f;
+      s += l[i];
+    }
+  } else {
+    float m = -INFINITY;
+    SLOTS(i) m = fmaxf(m, l[i]);
+    m = group_max<W>(m);
+    SLOTS(i) {
+      l[i] = (lane + W * i) < experts ? __expf(l[i] - m) : 0.0f;
+      s += l[i];
+    }
+  }
+  s = group_sum<W>(s);
+  SLOTS(i) l[i] /= s;
 }
 
 // Per-chunk partial column sums of the routing probabilities and per-chunk
@@ -296,27 +338,8 @@ __global__ void __launch_bounds__(256) router_stats_partial_kernel(
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       if (t0 + G * u >= end) break;  // uniform over the group
-      if (mode == MI355X_ROUTE_SIGMOID_NOAUX_TC) {
-        float s = 0.0f;
-        SLOTS(i) {
-          int e = lane + W * i;
-          l[u][i] = e < experts ? sigmoid_f(l[u][i]) : 0.0f;
-          s += l[u][i];
-        }
-        s = group_sum<W>(s);
-        SLOTS(i) acc[i] += l[u][i] / s;
-      } else {
-        float m = -INFINITY;
-        SLOTS(i) m = fmaxf(m, l[u][i]);
-        m = group_max<W>(m);
-        float s = 0.0f;
-        SLOTS(i) {
-          l[u][i] = (lane + W * i) < experts ? __expf(l[u][i] - m) : 0.0f;
-          s += l[u][i];
-        }
-        s = group_sum<W>(s);
-        SLOTS(i) acc[i] += l[u][i] / s;
-      }
+      token_probabilities<W, PL>(l[u], experts, mode);
+      SLOTS(i) acc[i] += l[u][i];
       if (id[u] >= 0) atomicAdd(&counts[id[u]], 1);
     }
   }
@@ -453,22 +476,20 @@ __global__ void __launch_bounds__(256) router_stats_pairs_kernel(
 // 2. Per expert: the segment sums into prob_sum and the aux loss terms, added
 //    over experts in a fixed order.
 constexpr int kAuxThreads = 512;
-__global__ void __launch_bounds__(kAuxThreads) router_stats_aux_kernel(
-    const float* __restrict__ part_p, int nchunks, int tokens, int experts, int top_k, int mode,
-    int segments, const int32_t* __restrict__ seg_offsets,
-    const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ seg_counts,
-    float* __restrict__ aux, float* __restrict__ prob_sum) {
-  __shared__ int seg_start[kReduceMaxSegments + 1];
-  __shared__ float red[kAuxThreads / 64];
-  segment_starts(chunk_table, nchunks, segments, seg_start);
+// The aux terms of experts first, first + kAuxThreads, ...; `sum_of` and
+// `count_of` give a (segment, expert) pair's probability sum and count.
+template <typename Sum, typename Count>
+__device__ __forceinline__ float aux_terms(int first, int tokens, int experts, int top_k, int mode,
+                                           int segments, const int32_t* __restrict__ seg_offsets,
+                                           Sum&& sum_of, Count&& count_of,
+                                           float* __restrict__ prob_sum) {
   float aux_part = 0.0f;
-  for (int e = threadIdx.x; e < experts; e += kAuxThreads) {
+  for (int e = first; e < experts; e += kAuxThreads) {
     float total_p = 0.0f;
     int total_c = 0;
     for (int s = 0; s < segments; ++s) {
-      const int c0 = seg_start[s];
-      const float sp = c0 < seg_start[s + 1] ? part_p[(size_t)c0 * experts + e] : 0.0f;
-      const int sc = seg_counts[(size_t)s * experts + e];
+      const float sp = sum_of(s * experts + e);
+      const int sc = count_of(s * experts + e);
       total_p += sp;
       total_c += sc;
       if (mode == MI355X_ROUTE_SIGMOID_NOAUX_TC) {
@@ -484,14 +505,190 @@ __global__ void __launch_bounds__(kAuxThreads) router_stats_aux_kernel(
       aux_part += freq * (total_p / (float)tokens);
     }
   }
-  aux_part = wave_sum(aux_part);
-  if (lane_id() == 0) red[threadIdx.x >> 6] = aux_part;
+  return aux_part;
+}
+__device__ __forceinline__ float aux_total(const float* red, int experts, int mode) {
+  float total = 0.0f;
+  for (int w = 0; w < kAuxThreads / 64; ++w) total += red[w];
+  return mode == MI355X_ROUTE_SIGMOID_NOAUX_TC ? total : (float)experts * total;
+}
+
+__global__ void __launch_bounds__(kAuxThreads) router_stats_aux_kernel(
+    const float* __restrict__ part_p, int nchunks, int tokens, int experts, int top_k, int mode,
+    int segments, const int32_t* __restrict__ seg_offsets,
+    const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ seg_counts,
+    float* __restrict__ aux, float* __restrict__ prob_sum) {
+  __shared__ int seg_start[kReduceMaxSegments + 1];
+  __shared__ float red[kAuxThreads / 64];
+  segment_starts(chunk_table, nchunks, segments, seg_start);
+  const float aux_part = aux_terms(
+      threadIdx.x, tokens, experts, top_k, mode, segments, seg_offsets,
+      [&](int p) {
+        const int s = p / experts, c0 = seg_start[s];
+        return c0 < seg_start[s + 1] ? part_p[(size_t)c0 * experts + p % experts] : 0.0f;
+      },
+      [&](int p) { return seg_counts[p]; }, prob_sum);
+  const float total = wave_sum(aux_part);
+  if (lane_id() == 0) red[threadIdx.x >> 6] = total;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float total = 0.0f;
-    for (int w = 0; w < kAuxThreads / 64; ++w) total += red[w];
-    aux[0] = mode == MI355X_ROUTE_SIGMOID_NOAUX_TC ? total : (float)experts * total;
+  if (threadIdx.x == 0) aux[0] = aux_total(red, experts, mode);
+}
+
+// Both in one block, for few chunks and pairs: the same sums in the same
+// order, the segment sums handed over in LDS. With the partial kernel 7.9 us
+// against 8.8 for the three at 509 tokens of 128 experts, 8.6 / 8.8 at 16
+// chunks, 10.4 / 8.9 at 32 (one CU then reads all the partials).
+constexpr int kFinishThreads = 1024, kFinishPairs = 1024, kFinishChunks = 16;
+__global__ void __launch_bounds__(kFinishThreads) router_stats_finish_kernel(
+    const float* __restrict__ part_p, const int32_t* __restrict__ part_c, int nchunks, int tokens,
+    int experts, int top_k, int mode, int segments, const int32_t* __restrict__ seg_offsets,
+    const int32_t* __restrict__ chunk_table, float* __restrict__ aux,
+    float* __restrict__ prob_sum, int32_t* __restrict__ seg_counts) {
+  __shared__ int seg_start[kFinishPairs + 1];
+  __shared__ float sums[kFinishPairs];
+  __shared__ int totals[kFinishPairs];
+  __shared__ float red[kAuxThreads / 64];
+  segment_starts(chunk_table, nchunks, segments, seg_start);
+  const int part = threadIdx.x % kPairLanes, pairs = segments * experts;
+  for (int pair = threadIdx.x / kPairLanes; pair < pairs; pair += kFinishThreads / kPairLanes) {
+    const int seg = pair / experts, e = pair % experts;
+    const int c_end = seg_start[seg + 1];
+    float sp = 0.0f;
+    int sc = 0;
+    for (int c = seg_start[seg] + part; c < c_end; c += kPairLanes) {
+      sp += part_p[(size_t)c * experts + e];
+      sc += part_c[(size_t)c * experts + e];
+    }
+    sp = group_sum<kPairLanes>(sp);
+#pragma unroll
+    for (int o = kPairLanes / 2; o >= 1; o >>= 1) sc += __shfl_xor(sc, o, 64);
+    if (part == 0) {
+      sums[pair] = sp;
+      totals[pair] = sc;
+      seg_counts[pair] = sc;
+    }
   }
+  __syncthreads();
+  if (threadIdx.x < kAuxThreads) {
+    const float part_sum = aux_terms(threadIdx.x, tokens, experts, top_k, mode, segments, seg_offsets,
+                                     [&](int p) { return sums[p]; }, [&](int p) { return totals[p]; },
+                                     prob_sum);
+    const float wave = wave_sum(part_sum);
+    if (lane_id() == 0) red[threadIdx.x >> 6] = wave;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) aux[0] = aux_total(red, experts, mode);
+}
+
+// Routing of at most 64 tokens (one statistics chunk, one segment; experts <=
+// 128, top_k <= 16, no group limit) in one block: top-k by 16-lane groups, the
+// statistics from probabilities in LDS, and the permutation plan, each in the
+// order of the separate kernels (bitwise the same). Seven launches of 2-5 us
+// kernels, most of a decode step's gaps, become one: 6.5 us against 19.8 for
+// one token of 128 experts, 11.9 against 22.8 for 61 (launch to launch).
+constexpr int kSmallTokens = kStatsChunk, kSmallThreads = 16 * kSmallTokens;
+template <int PL>
+__global__ void __launch_bounds__(kSmallThreads) route_small_kernel(
+    const float* __restrict__ logits, int tokens, int experts, int top_k, int mode,
+    const float* __restrict__ bias, float routed_scaling, const int32_t* __restrict__ forced,
+    float* __restrict__ weights, int32_t* __restrict__ ids, int64_t* __restrict__ counts,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ order, int32_t* __restrict__ slots,
+    float* __restrict__ aux, float* __restrict__ prob_sum) {
+  constexpr int W = 16, per_lane = PL, kWavesHere = kSmallThreads / 64;
+  __shared__ float prob[kSmallTokens][W * PL];
+  __shared__ int sid[kSmallTokens * kRowTopK];
+  __shared__ int count[kRowExperts], start[kRowExperts];
+  __shared__ uint8_t wave_count[kWavesHere][kRowExperts];
+  __shared__ float sums[kRowExperts], red[kAuxThreads / 64];
+  const int tid = threadIdx.x, lane = tid & (W - 1), token = tid / W, wave = tid >> 6;
+  if (tid < kRowExperts) count[tid] = 0;
+  for (int j = tid; j < kWavesHere * kRowExperts / 4; j += kSmallThreads)
+    ((uint32_t*)wave_count)[j] = 0;
+  __syncthreads();
+  if (token < tokens) {
+    float w;
+    int id;
+    topk_token<W, PL>(logits, token, experts, top_k, mode, bias, 1, 1, routed_scaling, forced,
+                      nullptr, w, id);
+    if (lane < top_k) {
+      const int flat = token * top_k + lane;
+      weights[flat] = w;
+      ids[flat] = id;
+      sid[flat] = id;
+      atomicAdd(&count[id], 1);
+    }
+    float l[kMaxPerLane];
+    SLOTS(i) {
+      const int e = lane + W * i;
+      l[i] = e < experts ? logits[(size_t)token * experts + e] : -INFINITY;
+    }
+    token_probabilities<W, PL>(l, experts, mode);
+    SLOTS(i) prob[token][lane + W * i] = l[i];
+  }
+  __syncthreads();
+  // Statistics: the partial kernel's 16 group sums (tokens q, q + 16, ...),
+  // added in group order.
+  if (tid < experts) {
+    float total = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      float acc = 0.0f;
+      for (int t = q; t < tokens; t += 16) acc += prob[t][tid];
+      total = q == 0 ? acc : total + acc;
+    }
+    sums[tid] = total;
+  }
+  // Plan: exclusive scan of the counts, two experts per lane of the last wave.
+  if (wave == kWavesHere - 1) {
+    const int e0 = 2 * lane_id();
+    const int c0 = e0 < experts ? count[e0] : 0, c1 = e0 + 1 < experts ? count[e0 + 1] : 0;
+    int x = c0 + c1;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane_id() >= o) x += y;
+    }
+    const int base = x - c0 - c1;
+    if (e0 < experts) {
+      start[e0] = base;
+      offsets[e0] = base;
+      counts[e0] = c0;
+    }
+    if (e0 + 1 < experts) {
+      start[e0 + 1] = base + c0;
+      offsets[e0 + 1] = base + c0;
+      counts[e0 + 1] = c1;
+    }
+    if (e0 == 0) offsets[experts] = tokens * top_k;
+  }
+  // Stable ranks: equal ids by wave, then by lane.
+  const int n = tokens * top_k;
+  const bool valid = tid < n;
+  const int e = valid ? sid[tid] : experts;
+  uint64_t peers = __ballot(1);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const uint64_t ones = __ballot((e >> b) & 1);
+    peers &= ((e >> b) & 1) ? ones : ~ones;
+  }
+  const int rank = __popcll(peers & lanes_below());
+  if (valid && rank == 0) wave_count[wave][e] = (uint8_t)__popcll(peers);
+  __syncthreads();
+  if (valid) {
+    int pos = start[e] + rank;
+    for (int w = 0; w < wave; ++w) pos += wave_count[w][e];
+    order[pos] = tid;
+    slots[tid] = pos;
+  }
+  if (tid < kAuxThreads) {
+    const float part_sum = aux_terms(tid, tokens, experts, top_k, mode, 1, nullptr,
+                                     [&](int p) { return sums[p]; }, [&](int p) { return count[p]; },
+                                     prob_sum);
+    const float total = wave_sum(part_sum);
+    if (lane_id() == 0) red[wave] = total;
+  }
+  __syncthreads();
+  if (tid == 0) aux[0] = aux_total(red, experts, mode);
 }
 
 template <int W, int PL>
@@ -707,10 +904,7 @@ template <int W, int PL> struct BwdK { static constexpr auto fn = router_bwd_ker
 
 }  // namespace
 
-extern "C" int mi355x_router_topk(const float* logits, int tokens, int experts, int top_k,
-                                  int mode, const float* bias, int n_group, int topk_group,
-                                  float routed_scaling, const int32_t* forced_ids,
-                                  float* weights, int32_t* ids, void* stream) {
+static int topk_checks(int tokens, int experts, int top_k, int mode, int n_group, int topk_group) {
   MI355X_REQUIRE(tokens >= 0 && experts > 0 && experts <= 64 * kMaxPerLane,
                  "router: experts must be in [1, %d], got %d", 64 * kMaxPerLane, experts);
   MI355X_REQUIRE(top_k > 0 && top_k <= experts && top_k <= kMaxTopK,
@@ -721,6 +915,15 @@ extern "C" int mi355x_router_topk(const float* logits, int tokens, int experts, 
                    "router: n_group must divide experts and be <= 64");
     MI355X_REQUIRE(topk_group > 0, "router: topk_group must be positive");
   }
+  return MI355X_OK;
+}
+
+extern "C" int mi355x_router_topk(const float* logits, int tokens, int experts, int top_k,
+                                  int mode, const float* bias, int n_group, int topk_group,
+                                  float routed_scaling, const int32_t* forced_ids,
+                                  float* weights, int32_t* ids, void* stream) {
+  const int c = topk_checks(tokens, experts, top_k, mode, n_group, topk_group);
+  if (c != MI355X_OK) return c;
   if (tokens == 0) return MI355X_OK;
   // Group-limited selection keeps a whole wavefront per token.
   const bool grouped = mode == MI355X_ROUTE_SIGMOID_NOAUX_TC && topk_group < n_group;
@@ -730,6 +933,31 @@ extern "C" int mi355x_router_topk(const float* logits, int tokens, int experts, 
                        (hipStream_t)stream, logits, tokens, experts, top_k, mode, bias, n_group,
                        topk_group, routed_scaling, forced_ids, weights, ids);
   });
+  MI355X_LAUNCH_CHECK();
+  return MI355X_OK;
+}
+
+// Top-k, plan and statistics in one launch; returns 1 outside its range.
+int mi355x_route_small(const float* logits, int tokens, int experts, int top_k, int mode,
+                       const float* bias, int n_group, int topk_group, float routed_scaling,
+                       const int32_t* forced_ids, int segments, float* weights, int32_t* ids,
+                       int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
+                       float* aux, float* prob_sum, void* stream) {
+  if (tokens < 1 || tokens > kSmallTokens || segments != 1 || experts > kRowExperts ||
+      top_k > kRowTopK || (mode == MI355X_ROUTE_SIGMOID_NOAUX_TC && topk_group < n_group))
+    return 1;
+  const int c = topk_checks(tokens, experts, top_k, mode, n_group, topk_group);
+  if (c != MI355X_OK) return c;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kSmallThreads), 0, (hipStream_t)stream, logits,
+                       tokens, experts, top_k, mode, bias, routed_scaling, forced_ids, weights,
+                       ids, counts, offsets, order, slots, aux, prob_sum);
+  };
+  const int need = (experts + 15) / 16;
+  if (need <= 1) launch(route_small_kernel<1>);
+  else if (need <= 2) launch(route_small_kernel<2>);
+  else if (need <= 4) launch(route_small_kernel<4>);
+  else launch(route_small_kernel<8>);
   MI355X_LAUNCH_CHECK();
   return MI355X_OK;
 }
@@ -765,8 +993,12 @@ extern "C" int mi355x_router_stats(const float* logits, const int32_t* ids, int 
                        mode, seg_offsets, chunk_table, part_p, part_c);
   });
   MI355X_LAUNCH_CHECK();
-  if (segments <= kReduceMaxSegments) {
-    const long long pairs = (long long)segments * experts;
+  const long long pairs = (long long)segments * experts;
+  if (nchunks <= kFinishChunks && pairs <= kFinishPairs) {
+    hipLaunchKernelGGL(router_stats_finish_kernel, dim3(1), dim3(kFinishThreads), 0, s, part_p,
+                       part_c, nchunks, tokens, experts, top_k, mode, segments, seg_offsets,
+                       chunk_table, aux, prob_sum, seg_counts);
+  } else if (segments <= kReduceMaxSegments) {
     const int per_block = 256 / kPairLanes;
     hipLaunchKernelGGL(router_stats_pairs_kernel, dim3((unsigned)((pairs + per_block - 1) / per_block)),
                        dim3(256), 0, s, part_p, part_c, nchunks, experts, segments, chunk_table,

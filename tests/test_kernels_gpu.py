@@ -206,6 +206,57 @@ def test_permute_quantize_bit_exact(device):
     assert torch.equal(s.cpu(), os_)
 
 
+@pytest.mark.parametrize("mode", ["topk_then_softmax", "softmax_then_topk", "sigmoid_noaux_tc"])
+@pytest.mark.parametrize("tokens,experts,top_k", [
+    (1, 128, 8), (1, 1, 1), (16, 16, 2), (17, 33, 16), (63, 127, 5), (64, 128, 16),
+    (65, 128, 8),            # two statistics chunks: the separate kernels
+    (64, 129, 4), (64, 128, 17),
+])
+def test_route_in_one_launch_equals_separate_kernels(device, mode, tokens, experts, top_k):
+    """Top-k, statistics and plan fused for few tokens, at the edges of its
+    range: bitwise the separate kernels, with a bias, NaN, infinities and ties
+    among the logits, and forced ids."""
+    g = torch.Generator().manual_seed(tokens * experts + top_k)
+    logits = torch.randn(tokens, experts, generator=g)
+    logits[:, experts // 2] = logits[:, 0]
+    logits[0, experts - 1] = float("inf") if top_k < experts else 0.0
+    if tokens > 2:
+        logits[1, 0] = -float("inf")
+        logits[2] = 0.0
+    if tokens > 16:
+        logits[16, experts // 3] = float("nan")
+    logits = logits.to(device)
+    bias = (torch.randn(experts, generator=g) * 0.1).to(device)
+    forced = torch.stack([torch.randperm(experts, generator=g)[:top_k]
+                          for _ in range(tokens)]).to(torch.int32).to(device)
+    for forced_ids in (None, forced):
+        options = dict(bias=bias if mode == "sigmoid_noaux_tc" else None, routed_scaling=2.5,
+                       forced_ids=forced_ids)
+        got = K.route(logits, top_k, mode, (tokens,), **options)
+        weights, ids = K.router_topk(logits, top_k, mode, **options)
+        aux, prob_sum, _, _ = K.router_stats(logits, ids, top_k, mode, (tokens,))
+        want = (weights, ids, *K.permute_plan(ids, experts), aux, prob_sum)
+        for a, b in zip(got, want, strict=True):
+            assert a.dtype == b.dtype and torch.equal(_bytes(a.reshape(-1)), _bytes(b.reshape(-1)))
+
+
+@pytest.mark.parametrize("assignments,experts", [(1, 1), (1024, 300), (1025, 1024), (6144, 128),
+                                                 (6145, 128)])
+def test_permute_plan_around_the_one_block_size(device, assignments, experts):
+    """The plan in one block (up to 6144 assignments) and in three kernels
+    against the oracle's stable sort, with an overloaded and an empty expert."""
+    g = torch.Generator().manual_seed(assignments)
+    ids = torch.randint(0, experts, (assignments, 1), generator=g)
+    ids[torch.rand(assignments, generator=g) < 0.3] = 0
+    ids[ids == experts - 1] = 0
+    ids = ids.to(torch.int32)
+    counts, offsets, order, slots = K.permute_plan(ids.to(device), experts)
+    want_order, want_offsets, want_slots = O.sort_assignments(ids, experts)
+    assert torch.equal(order.cpu(), want_order) and torch.equal(offsets.cpu(), want_offsets)
+    assert torch.equal(slots.cpu(), want_slots)
+    assert torch.equal(counts.cpu(), torch.bincount(ids.reshape(-1).long(), minlength=experts))
+
+
 @pytest.mark.parametrize("gate_up", [False, True])
 def test_quantize_rows_bit_exact(device, gate_up):
     g = torch.Generator().manual_seed(15)

@@ -552,6 +552,8 @@ def test_gathered_token_rows_equal_permuted_copy_in_the_layer(device, monkeypatc
     ("fp8_block", 97, 64, 8, 256, "softmax_then_topk"),      # router gradient on its kernel
     ("fp8_block", 130, 8, 3, 384, "sigmoid_noaux_tc"),       # w2's transposed copy, sequences
     ("fp8_current", 65, 16, 4, 256, "topk_then_softmax"),
+    ("fp8_block", 64, 128, 16, 256, "softmax_then_topk"),    # the fused routing's largest call
+    ("fp8_block", 17, 40, 5, 256, "sigmoid_noaux_tc"),       # and odd sizes
 ])
 def test_launch_sequences_equal_single_kernel_calls(device, precision, tokens, experts, top_k,
                                                     inter, mode):
@@ -559,7 +561,7 @@ def test_launch_sequences_equal_single_kernel_calls(device, precision, tokens, e
     called one at a time (as they are while a launch timer is installed)."""
     x, res, wr, w13, w2, dy = _inputs(device, tokens=tokens, hidden=256, experts=experts,
                                       inter=inter, seed=13)
-    lengths = (tokens // 2, tokens - tokens // 2) if mode == "sigmoid_noaux_tc" else None
+    lengths = (tokens // 2, tokens - tokens // 2) if tokens == 130 else None
 
     def run():
         leaves = [t.clone().requires_grad_(True) for t in (x, wr, w13, w2)]
