@@ -45,9 +45,11 @@ __device__ __forceinline__ int swz(int row) { return row & 7; }
 // compiler's wait-count bookkeeping: it would otherwise wait for every
 // in-flight load before any LDS read it cannot prove disjoint. The kernels
 // count their own loads and wait with wait_and_sync<N>.
-// LDS byte address of a (wave-uniform) LDS pointer, as a scalar for M0.
+// LDS byte address of a (wave-uniform) LDS pointer, as a scalar for M0: the
+// low half of the generic address (a cast to an LDS pointer would also test
+// it for null, where the compiler cannot prove that it is none).
 __device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(lds_ptr_t)p);
+  return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)p);
 }
 // Source address = wave-uniform 64-bit base (SGPRs) + per-lane 32-bit byte
 // offset (one VGPR), the saddr form of the global load.

@@ -151,14 +151,17 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     const size_t koff = (size_t)kb * BK;
     const uint8_t* abase = a + koff;
     const uint8_t* bbase = w + (size_t)t.e * N * K + koff;
+    // A wave whose 32 rows lie past the tile's rows copies none of them.
+    if (wave * (8 * A_LOADS) < t.nvalid) {
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
-      const int r = (wave * A_LOADS + i) * 8 + (lane >> 3);
-      int src;
-      if constexpr (kGather) src = (int)div_rows((uint32_t)gtok[t.par][r], div_m, div_s);
-      else src = min(t.row0 + r, rows - 1);
-      const uint32_t off = (uint32_t)src * (uint32_t)K + 16 * ((lane & 7) ^ swz(r));
-      dma16(abase, off, base + (wave * A_LOADS + i) * 1024);
+      for (int i = 0; i < A_LOADS; ++i) {
+        const int r = (wave * A_LOADS + i) * 8 + (lane >> 3);
+        int src;
+        if constexpr (kGather) src = (int)div_rows((uint32_t)gtok[t.par][r], div_m, div_s);
+        else src = min(t.row0 + r, rows - 1);
+        const uint32_t off = (uint32_t)src * (uint32_t)K + 16 * ((lane & 7) ^ swz(r));
+        dma16(abase, off, base + (wave * A_LOADS + i) * 1024);
+      }
     }
     if constexpr (kKM) {
       // K rows kb*128 .. +127 of the expert's [K, N] weight, columns of the
@@ -291,6 +294,17 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
       }
     }
 
+    // A wave whose 64 rows lie past the tile's rows (the last row block of an
+    // expert) only copies weights: waves w and w + 4 share a SIMD and hold the
+    // two halves of the tile, so a block of up to 128 rows costs half the
+    // MFMAs and 3/4 of the copies. Half of the experts end in such a block.
+    // Measured us, before / after: hidden 7168, 2048, 32 experts at 16384 rows
+    // up 740 / 695, down 346 / 315, row-scaled up 603 / 552; hidden 2048, 768,
+    // 128 experts at 32744 rows up 202 / 185, down 113 / 98, at 131072 rows up
+    // 542 / 523, down 293 / 282. (Such blocks at the end of the list, behind
+    // all full ones, balance the CUs better but read their weights a second
+    // time: no faster.)
+    const bool active = wm * 64 < ct.nvalid;
     for (int kb = 0; kb < nk; ++kb) {
       wait_and_sync<0>();  // two stages: the only loads in flight are this step's
       if (kGather && kb == 0 && next_tile < total) {
@@ -308,7 +322,7 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
       // block instead, so that while one wave of a SIMD is held the other
       // has MFMAs to issue. (A later issue point needs registers the step
       // does not have: the compiler spills.)
-      const bool late = wave >= 4 && kb + 1 < nk;
+      const bool late = wave >= 4 && active && kb + 1 < nk;
       if (late) {
         // issued in the K step below, at MFMA block kLateIssueBlock
       } else if (kb + 1 < nk) {
@@ -317,6 +331,10 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
         Tile nt = describe(prefix, offsets, experts, n_tiles, next_tile, nk, n_group, rotate);
         if constexpr (kGather) nt.par = (round + 1) & 1;
         issue(nt, 0, stage ^ 1);
+      }
+      if (!active) {
+        stage ^= 1;
+        continue;
       }
       const uint8_t* base = smem + stage * STAGE_BYTES;
       const uint8_t* ta = base;

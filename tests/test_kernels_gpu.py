@@ -426,6 +426,8 @@ TILE_CASES = [
     ([129, 160, 256, 1, 250], 256, 640),
     ([129, 160, 256, 1, 250], 384, 384),
     ([300, 511, 0, 900], 4096, 256),
+    # 256 x 256 tiles with 1 to 4 of their 64-row groups in use, around each edge.
+    ([257, 64, 321, 128, 129, 448, 705, 0, 255], 4096, 384),
     ([300, 511, 0, 900], 12416, 128),
 ]
 
