@@ -481,6 +481,32 @@ int mi355x_gemm_fp8_block_swiglu(const uint8_t* a, const float* a_scale, int row
                                  int k, const int32_t* offsets, const void* addend, float limit,
                                  void* h, uint8_t* act_q, float* act_scales, void* stream);
 
+/* Any form of the grouped GEMM above except the fused SwiGLU, from one
+ * argument struct, with scratch for its last round of tiles. Where that round
+ * would occupy few of the CUs for a long K, the launch splits it over K into
+ * `workspace` (mi355x_gemm_tail_workspace_size bytes; 0: this shape never
+ * does) and adds the fp32 parts in a fixed order in a second launch; without
+ * a workspace it equals the entry points above. Unused fields are zero;
+ * a_rows_div is 1 unless a_rows is given. */
+typedef struct mi355x_gemm_args {
+  const uint8_t* a;        /* [rows, K], or [a_total, K] with a_rows */
+  const float* a_scale;    /* as the form's own entry point takes them */
+  const int32_t* a_rows;   /* gathered forms, else NULL */
+  const uint8_t* w;        /* [E, N, K], or [E, K, N] with kmajor */
+  const float* w_scale;
+  const int32_t* offsets;  /* [E + 1] */
+  const void* addend;      /* bf16 [rows, N] or NULL */
+  const void* lora_z;      /* with lora_rank, else NULL */
+  const void* lora_b;
+  void* out;               /* bf16 [rows, N] */
+  void* workspace;         /* or NULL */
+  uint64_t workspace_bytes;
+  int32_t rows, a_total, a_rows_div, experts, n, k;
+  int32_t w_scale_t, interleave, row_scaled, kmajor, lora_rank;
+} mi355x_gemm_args;
+size_t mi355x_gemm_tail_workspace_size(int rows, int experts, int n, int k);
+int mi355x_gemm_fp8(const mi355x_gemm_args* args, void* stream);
+
 /* Grouped weight-gradient GEMM over feature-major e4m3 operands of the same
  * padded layout (see mi355x_quantize_transpose_fp8):
  *   out[e][m][n] = sum_{rows of e} p[m][row] q[n][row], block-scaled,
@@ -515,7 +541,7 @@ int mi355x_moe_route(const float* logits, int tokens, int experts, int top_k, in
                      int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
                      float* aux, float* prob_sum, void* workspace, size_t workspace_bytes,
                      void* stream);
-size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter);
+size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter, int experts);
 int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidden, int inter, float limit,
                     int row_scaled, const uint8_t* w2, const float* w2_scale, int experts,
                     const int32_t* offsets, const int32_t* slots, const float* weights,

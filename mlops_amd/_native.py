@@ -101,11 +101,13 @@ SIGNATURES = {
     "mi355x_moe_route_workspace_size": (_S, [_I, _I, _I, _I, _I]),
     "mi355x_moe_route": (_I, [_P, _I, _I, _I, _I, _P, _I, _I, _F, _P, _I, _P, _P, _I, _P, _P, _P,
                               _P, _P, _P, _P, _P, _P, _S, _P]),
-    "mi355x_moe_down_workspace_size": (_S, [_I, _I, _I]),
+    "mi355x_moe_down_workspace_size": (_S, [_I] * 4),
     "mi355x_moe_down": (_I, [_P, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _S,
                              _P]),
     "mi355x_moe_block_bwd_workspace_size": (_S, [_I] * 8),
     "mi355x_moe_block_bwd": (_I, [ctypes.c_char_p, _P]),  # the packed argument struct
+    "mi355x_gemm_tail_workspace_size": (_S, [_I] * 4),
+    "mi355x_gemm_fp8": (_I, [ctypes.c_char_p, _P]),  # the packed argument struct
 }
 
 _lock = threading.Lock()

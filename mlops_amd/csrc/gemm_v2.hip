@@ -23,7 +23,35 @@ struct Tile {
   int e, row0, nvalid, nt;
   int rot;  // K-step rotation: the tile walks K steps rot, rot + 1, ... (mod nk)
   int par;  // which of the two gathered-row tables holds this tile's A rows
+  int steps;  // K steps: all of them, or those of one part of a split tile
 };
+
+// The last round of an XCD's tiles leaves CUs idle: `rest` tiles for `cus` of
+// them. Given scratch, the round is split over K: part p of `parts` of tile t
+// runs on CU p * rest + t and writes its fp32 accumulators, and a second
+// launch (Phase::kFinish) adds the parts in order and stores the tile. Worth
+// it where the steps this takes off the round outweigh the parts' way through
+// memory and the second launch (256 KB a CU, 30-40 us against 2.6 us a step).
+// Measured us, whole / split: hidden 4096, 14336, 8 experts at 4096 rows
+// (320 tiles, 40 an XCD) down 388 / 301, dx 767 / 608, row-scaled down 366 /
+// 274; at 8192 rows 583 / 518, 1230 / 1063, 541 / 455. Whole parts, so that
+// the CUs of a part walk the same K steps and share operand panels in L2:
+// the round's steps dealt evenly to all CUs, across tile borders, lost that
+// (hidden 7168, 2048, 32 experts at 16384 rows up 660 whole, 697 so).
+struct Tail {
+  int full_rounds, rest;
+  int parts;  // 1: the last round runs whole tiles
+};
+constexpr int kMinPartSteps = 8, kMinSavedSteps = 24;
+
+__host__ __device__ inline Tail tail_split(int tiles, int cus, int nk) {
+  Tail t = {tiles / cus, tiles % cus, 1};
+  if (t.rest > 0 && 2 * t.rest <= cus && nk >= 2 * kMinPartSteps) {
+    t.parts = cus / t.rest < nk / kMinPartSteps ? cus / t.rest : nk / kMinPartSteps;
+    if (nk - (nk + t.parts - 1) / t.parts < kMinSavedSteps) t.parts = 1;
+  }
+  return t;
+}
 
 __device__ __forceinline__ Tile describe(const int* prefix, const int32_t* __restrict__ offsets,
                                          int experts, int n_tiles, int tile, int nk, int n_group,
@@ -62,6 +90,7 @@ __device__ __forceinline__ Tile describe(const int* prefix, const int32_t* __res
   // together.
   t.rot = rotate ? __builtin_amdgcn_readfirstlane(nk >= 8 ? tile % 3 : (tile * 7) % nk) : 0;
   t.par = 0;
+  t.steps = nk;
   return t;
 }
 
@@ -93,8 +122,11 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 // MFMA block of a K step at which waves 4-7 issue the next step's copies.
 constexpr int kLateIssueBlock = 1;
 
+// kPhase: what a launch does about its last round of tiles (see tail_split).
+enum class Phase { kWhole, kSplit, kFinish };
+
 template <bool kAct, bool kAdd, bool kLora, bool kRow = false, bool kKM = false,
-          bool kGather = false>
+          bool kGather = false, Phase kPhase = Phase::kWhole>
 __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ a_scale, int rows,
     const uint8_t* __restrict__ w, const float* __restrict__ w_scale, int w_scale_t, int experts,
@@ -102,8 +134,9 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     const uint16_t* __restrict__ addend, uint16_t* __restrict__ out,
     uint8_t* __restrict__ act_q, float* __restrict__ act_scales, float limit,
     const uint16_t* __restrict__ lora_z, const uint16_t* __restrict__ lora_b, int lora_rank,
-    int n_group, int rotate, const int32_t* __restrict__ a_rows, int scale_pitch,
-    uint32_t div_m, int div_s) {
+    int n_group, int rotate, const int32_t* __restrict__ a_rows, uint32_t div_m, int div_s,
+    float* __restrict__ partial) {
+  static_assert(!kAct || kPhase == Phase::kWhole, "the fused SwiGLU takes whole tiles");
   __shared__ __align__(1024) uint8_t smem[kStages * STAGE_BYTES];
   __shared__ float act_amax[2][BM];  // per-row amax of each wave column's 64 act columns
   __shared__ int prefix[kMaxExperts + 1];
@@ -217,15 +250,42 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
   const int xcd = blockIdx.x & 7, cu = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
   const int first = affine ? (int)((long long)total * xcd / 8) : 0;
   const int last = affine ? (int)((long long)total * (xcd + 1) / 8) : total;
+  Tail tail = {0, 0, 1};
+  if constexpr (kPhase != Phase::kWhole) {
+    if (affine) tail = tail_split(last - first, per_xcd, nk);
+    if (kPhase == Phase::kFinish && tail.parts == 1) return;
+  }
+  // Round r is the split one (the last, so its tile has no successor).
+  auto split_at = [&](int r) -> bool {
+    return kPhase != Phase::kWhole && tail.parts > 1 && r == tail.full_rounds;
+  };
+  const int part = split_at(tail.full_rounds) ? cu / tail.rest : 0;
   auto tile_at = [&](int r) -> int {
     if (!affine) return tile_of(r, blockIdx.x, gridDim.x);
+    if (split_at(r))
+      return part < tail.parts ? first + r * per_xcd + cu - part * tail.rest : total;
     const int t = first + r * per_xcd + cu;
     return t < last ? t : total;
   };
-  int round = 0;
-  int tile = tile_at(0);
+  auto describe_at = [&](int r, int index) -> Tile {
+    Tile t = describe(prefix, offsets, experts, n_tiles, index, nk, n_group, rotate);
+    if (kPhase == Phase::kSplit && split_at(r)) {
+      t.rot = __builtin_amdgcn_readfirstlane(nk * part / tail.parts);
+      t.steps = __builtin_amdgcn_readfirstlane(nk * (part + 1) / tail.parts) - t.rot;
+    }
+    return t;
+  };
+  // A block's partial sums: MFMA block (i, jb) of all its threads together.
+  // Wave-uniform base + the thread's offset, through an empty asm at its use
+  // (32 hoisted addresses would spill inside the K loop).
+  auto partial_at = [&](int block, int i, int jb, uint32_t offset) -> v4f* {
+    return (v4f*)((uint8_t*)(partial + (size_t)block * (BM * BN) +
+                             (i * 8 + jb) * (4 * kThreads)) + offset);
+  };
+  int round = kPhase == Phase::kFinish ? tail.full_rounds : 0;
+  int tile = tile_at(round);
   if (tile >= total) return;
-  Tile ct = describe(prefix, offsets, experts, n_tiles, tile, nk, n_group, rotate);
+  Tile ct = describe_at(round, tile);
   // Gathered A: the tile's 256 source rows (row indices clamped to the last
   // row, as the plain copies clamp) into table `par`, by the first four waves'
   // direct loads; they land before the next wait_and_sync<0> returns.
@@ -238,7 +298,7 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     load_rows(ct, 0);
     wait_and_sync<0>();
   }
-  issue(ct, 0, 0);
+  if constexpr (kPhase != Phase::kFinish) issue(ct, 0, 0);
   int stage = 0;
   for (;;) {
     const int next_tile = tile_at(round + 1);
@@ -247,7 +307,7 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    if constexpr (kLora) {
+    if (kLora && kPhase != Phase::kFinish && !(split_at(round) && part > 0)) {
       // The accumulators start from the rank-r product z[row] . b[e][col]
       // (bf16 MFMA, fp32 sums, 16 of the rank at a time): the low-rank term
       // of out = A W^T + z B^T joins before the block products, with no
@@ -305,15 +365,14 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     // all full ones, balance the CUs better but read their weights a second
     // time: no faster.)
     const bool active = wm * 64 < ct.nvalid;
-    for (int kb = 0; kb < nk; ++kb) {
+    for (int kb = 0; kPhase != Phase::kFinish && kb < ct.steps; ++kb) {
       wait_and_sync<0>();  // two stages: the only loads in flight are this step's
       if (kGather && kb == 0 && next_tile < total) {
         // The next tile's source rows, into the other table (its last reader,
         // the tile before this one, finished before the barrier above). With
         // a single K step they are needed right away.
-        load_rows(describe(prefix, offsets, experts, n_tiles, next_tile, nk, n_group, rotate),
-                  (round + 1) & 1);
-        if (nk == 1) wait_and_sync<0>();
+        load_rows(describe_at(round + 1, next_tile), (round + 1) & 1);
+        if (ct.steps == 1) wait_and_sync<0>();
       }
       // Next step's operands (the next tile's first step at the last step:
       // its loads then run under this tile's epilogue). A wave is held at
@@ -322,13 +381,13 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
       // block instead, so that while one wave of a SIMD is held the other
       // has MFMAs to issue. (A later issue point needs registers the step
       // does not have: the compiler spills.)
-      const bool late = wave >= 4 && active && kb + 1 < nk;
+      const bool late = wave >= 4 && active && kb + 1 < ct.steps;
       if (late) {
         // issued in the K step below, at MFMA block kLateIssueBlock
-      } else if (kb + 1 < nk) {
+      } else if (kb + 1 < ct.steps) {
         issue(ct, kb + 1, stage ^ 1);
       } else if (next_tile < total) {
-        Tile nt = describe(prefix, offsets, experts, n_tiles, next_tile, nk, n_group, rotate);
+        Tile nt = describe_at(round + 1, next_tile);
         if constexpr (kGather) nt.par = (round + 1) & 1;
         issue(nt, 0, stage ^ 1);
       }
@@ -408,6 +467,31 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
         bcur = bnext;
       }
       stage ^= 1;
+    }
+
+    if (kPhase == Phase::kSplit && split_at(round)) {
+      if (active) {
+        uint32_t offset = 16 * tid;
+        asm volatile("" : "+v"(offset));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int jb = 0; jb < 8; ++jb) *partial_at(blockIdx.x, i, jb, offset) = acc[i][jb];
+      }
+      return;
+    }
+    if constexpr (kPhase == Phase::kFinish) {
+      // The tile's wave rows are dealt to the blocks that computed its parts.
+      if (wm % tail.parts != part) ct.nvalid = 0;
+      if (wm * 64 < ct.nvalid) {
+        for (int p = 0; p < tail.parts; ++p) {
+          const int block = (cu + (p - part) * tail.rest) * 8 + xcd;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int jb = 0; jb < 8; ++jb) acc[i][jb] += *partial_at(block, i, jb, 16 * tid);
+        }
+      }
     }
 
     // ---- epilogue straight from registers: lane (row, 8 consecutive
@@ -582,12 +666,10 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     if (next_tile >= total) break;
     ++round;
     tile = next_tile;
-    ct = describe(prefix, offsets, experts, n_tiles, tile, nk, n_group, rotate);
+    ct = describe_at(round, tile);
     if constexpr (kGather) ct.par = round & 1;
   }
 }
-
-}  // namespace
 
 // Tile order by the size of one expert's weight (N x K bytes). Up to a few
 // L2s' worth, tiles go row-block-major with the K rotation: an XCD's CUs
@@ -598,7 +680,6 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
 // together. Measured on MI355X: Mixtral's four GEMMs (58-117 MB per
 // expert) +6-14%, DeepSeek-shard up/dgrad-up (29 MB) +5-7%; the 3-15 MB
 // weights of the other shapes lose 1-7% in that order.
-namespace {
 struct Order {
   int n_group, rotate;
 };
@@ -606,16 +687,87 @@ Order tile_order(int n, int k) {
   if ((size_t)n * (size_t)k >= ((size_t)24 << 20)) return {8, 0};
   return {0, 1};
 }
+
+struct V2Args {
+  const uint8_t* a;
+  const float* a_scale;
+  int rows;
+  const uint8_t* w;
+  const float* w_scale;
+  int w_scale_t, experts, n, k;
+  const int32_t* offsets;
+  int interleave;
+  const void* addend;
+  void* out;
+  uint8_t* act_q;
+  float* act_scales;
+  float limit;
+  const void *lora_z, *lora_b;
+  int lora_rank;
+  const int32_t* a_rows;
+  int a_rows_div;
+  float* partial;  // mi355x_gemm_tail_workspace_size bytes, or null: whole tiles only
+};
+
+template <bool kAct, bool kAdd, bool kLora, bool kRow, bool kKM, bool kGather, Phase kPhase>
+void enqueue(const V2Args& g, int grid, hipStream_t stream) {
+  const Order order = tile_order(g.n, g.k);
+  const RowDiv div = row_div_magic(g.a_rows_div);
+  hipLaunchKernelGGL((grouped_gemm_v2_kernel<kAct, kAdd, kLora, kRow, kKM, kGather, kPhase>),
+                     dim3(grid), dim3(kThreads), 0, stream, g.a, g.a_scale, g.rows, g.w, g.w_scale,
+                     g.w_scale_t, g.experts, g.n, g.k, g.offsets, g.interleave,
+                     (const uint16_t*)g.addend, (uint16_t*)g.out, g.act_q, g.act_scales, g.limit,
+                     (const uint16_t*)g.lora_z, (const uint16_t*)g.lora_b, g.lora_rank,
+                     order.n_group, order.rotate, g.a_rows, div.m, div.s, g.partial);
+}
+
+template <bool kAct, bool kAdd, bool kLora, bool kRow = false, bool kKM = false,
+          bool kGather = false>
+int launch(const V2Args& g, void* stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const int cus = cu_count();
+  if constexpr (!kAct) {
+    if (g.partial != nullptr) {
+      enqueue<kAct, kAdd, kLora, kRow, kKM, kGather, Phase::kSplit>(g, cus, s);
+      MI355X_LAUNCH_CHECK();
+      enqueue<kAct, kAdd, kLora, kRow, kKM, kGather, Phase::kFinish>(g, cus, s);
+      MI355X_LAUNCH_CHECK();
+      return 0;
+    }
+  }
+  const int upper = ((g.rows + BM - 1) / BM + g.experts) * (g.n / BN);
+  enqueue<kAct, kAdd, kLora, kRow, kKM, kGather, Phase::kWhole>(g, upper < cus ? upper : cus, s);
+  MI355X_LAUNCH_CHECK();
+  return 0;
+}
+
 }  // namespace
 
+// Scratch for the split last round, 0 where a launch on `rows` rows is not
+// expected to have one: smaller tiles, a short K, or by the row blocks that
+// `rows` rows make on average no short last round (a second launch that finds
+// nothing to finish costs 4-6 us: hidden 4096, 14336, 8 experts at 2048 rows
+// down 201 / 207). Past ten rounds the last one is too small a share.
+extern "C" size_t mi355x_gemm_tail_workspace_size(int rows, int experts, int n, int k) {
+  if (rows <= 0 || experts <= 0 || experts > kMaxExperts || n <= 0 || n % BN != 0 || k <= 0 ||
+      k % BK != 0)
+    return 0;
+  const int cus = cu_count();
+  if (cus % 8 != 0 || mi355x_gemm_tile_serves(rows, experts, n)) return 0;
+  const int groups = rows < experts ? rows : experts;
+  const long long tiles = ((long long)rows / BM + groups / 2) * (n / BN);
+  if (tiles > 10ll * cus || tail_split((int)(tiles / 8), cus / 8, k / BK).parts == 1) return 0;
+  return (size_t)cus * BM * BN * sizeof(float);
+}
+
 // Launches the pipelined kernel; returns 1 if the shape is not its form
-// (N % 256 != 0), in which case the caller uses the general kernel.
+// (N % 256 != 0).
 int mi355x_gemm_v2_launch(const uint8_t* a, const float* a_scale, int rows, const uint8_t* w,
                           const float* w_scale, int w_scale_t, int experts, int n, int k,
                           const int32_t* offsets, int interleave, const void* addend, void* out,
                           uint8_t* act_q, float* act_scales, float limit, const void* lora_z,
-                          const void* lora_b, int lora_rank, void* stream,
-                          const int32_t* a_rows, int a_total, int a_rows_div) {
+                          const void* lora_b, int lora_rank, void* stream, const int32_t* a_rows,
+                          int a_rows_div, float* partial) {
   if (act_q == nullptr) {
     const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, w_scale_t, experts, n,
                                               k, offsets, interleave, addend, lora_z, lora_b,
@@ -626,32 +778,20 @@ int mi355x_gemm_v2_launch(const uint8_t* a, const float* a_scale, int rows, cons
     return 1;  // the caller runs the GEMM, then the SwiGLU pass: the same bytes
   }
   if (n % BN != 0 || experts > kMaxExperts || (interleave && (n / 2) % 128 != 0)) return 1;
-  const RowDiv div = row_div_magic(a_rows_div);
-  const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);
-  const int grid = upper < cu_count() ? upper : cu_count();
-  const Order order = tile_order(n, k);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, a, a_scale,
-                       rows, w, w_scale, w_scale_t, experts, n, k, offsets, interleave,
-                       (const uint16_t*)addend, (uint16_t*)out, act_q, act_scales, limit,
-                       (const uint16_t*)lora_z, (const uint16_t*)lora_b, lora_rank,
-                       order.n_group, order.rotate, a_rows, a_rows != nullptr ? a_total : rows, div.m, div.s);
-  };
+  const V2Args g = {a, a_scale, rows, w, w_scale, w_scale_t, experts, n, k, offsets, interleave,
+                    addend, out, act_q, act_scales, limit, lora_z, lora_b, lora_rank, a_rows,
+                    a_rows_div, partial};
+  const bool act = act_q != nullptr, add = addend != nullptr;
   if (a_rows != nullptr) {
-    if (lora_z != nullptr || act_q != nullptr || addend != nullptr) return 1;
-    launch(grouped_gemm_v2_kernel<false, false, false, false, false, true>);
-  } else if (lora_z != nullptr) {
-    if (act_q != nullptr || addend != nullptr) return 1;  // not a form of this kernel
-    launch(grouped_gemm_v2_kernel<false, false, true>);
-  } else if (act_q != nullptr) {
-    addend != nullptr ? launch(grouped_gemm_v2_kernel<true, true, false>)
-                      : launch(grouped_gemm_v2_kernel<true, false, false>);
-  } else {
-    addend != nullptr ? launch(grouped_gemm_v2_kernel<false, true, false>)
-                      : launch(grouped_gemm_v2_kernel<false, false, false>);
+    if (lora_z != nullptr || act || add) return 1;
+    return launch<false, false, false, false, false, true>(g, stream);
   }
-  MI355X_LAUNCH_CHECK();
-  return 0;
+  if (lora_z != nullptr) {
+    if (act || add) return 1;  // not a form of this kernel
+    return launch<false, false, true>(g, stream);
+  }
+  if (act) return add ? launch<true, true, false>(g, stream) : launch<true, false, false>(g, stream);
+  return add ? launch<false, true, false>(g, stream) : launch<false, false, false>(g, stream);
 }
 
 // K-major weight (see kKM): w [E, K, N] e4m3 with its own block scales
@@ -659,27 +799,16 @@ int mi355x_gemm_v2_launch(const uint8_t* a, const float* a_scale, int rows, cons
 int mi355x_gemm_v2_kmajor_launch(const uint8_t* a, const float* a_scale, int rows,
                                  const uint8_t* w, const float* w_scale, int experts, int n, int k,
                                  const int32_t* offsets, void* out, void* stream,
-                                 const int32_t* a_rows, int a_total, int a_rows_div) {
+                                 const int32_t* a_rows, int a_rows_div, float* partial) {
   const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, 1, experts, n, k,
                                             offsets, 0, nullptr, nullptr, nullptr, 0, out, a_rows,
                                             a_rows_div, false, true, stream);
   if (small <= 0) return small;
   if (n % BN != 0 || experts > kMaxExperts) return 1;
-  const RowDiv div = row_div_magic(a_rows_div);
-  const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);
-  const int grid = upper < cu_count() ? upper : cu_count();
-  const Order order = tile_order(n, k);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, a, a_scale,
-                       rows, w, w_scale, 1, experts, n, k, offsets, 0, (const uint16_t*)nullptr,
-                       (uint16_t*)out, (uint8_t*)nullptr, (float*)nullptr, 0.0f,
-                       (const uint16_t*)nullptr, (const uint16_t*)nullptr, 0, order.n_group,
-                       order.rotate, a_rows, a_rows != nullptr ? a_total : rows, div.m, div.s);
-  };
-  if (a_rows != nullptr) launch(grouped_gemm_v2_kernel<false, false, false, false, true, true>);
-  else launch(grouped_gemm_v2_kernel<false, false, false, false, true>);
-  MI355X_LAUNCH_CHECK();
-  return 0;
+  const V2Args g = {a, a_scale, rows, w, w_scale, 1, experts, n, k, offsets, 0, nullptr, out,
+                    nullptr, nullptr, 0.0f, nullptr, nullptr, 0, a_rows, a_rows_div, partial};
+  return a_rows != nullptr ? launch<false, false, false, false, true, true>(g, stream)
+                           : launch<false, false, false, false, true>(g, stream);
 }
 
 // Row-scaled form (see kRow): a_scale [rows], w_scale [E, N]; returns 1 if
@@ -688,28 +817,18 @@ int mi355x_gemm_v2_rowwise_launch(const uint8_t* a, const float* a_scale, int ro
                                   const uint8_t* w, const float* w_scale, int experts, int n,
                                   int k, const int32_t* offsets, const void* lora_z,
                                   const void* lora_b, int lora_rank, void* out, void* stream,
-                                  const int32_t* a_rows, int a_total, int a_rows_div) {
+                                  const int32_t* a_rows, int a_rows_div, float* partial) {
   const int small = mi355x_gemm_tile_launch(a, a_scale, rows, w, w_scale, 0, experts, n, k,
                                             offsets, 0, nullptr, lora_z, lora_b, lora_rank, out,
                                             a_rows, a_rows_div, true, false, stream);
   if (small <= 0) return small;
   if (n % BN != 0 || experts > kMaxExperts) return 1;
-  const RowDiv div = row_div_magic(a_rows_div);
-  const int upper = ((rows + BM - 1) / BM + experts) * (n / BN);
-  const int grid = upper < cu_count() ? upper : cu_count();
-  const Order order = tile_order(n, k);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, a, a_scale,
-                       rows, w, w_scale, 0, experts, n, k, offsets, 0, (const uint16_t*)nullptr,
-                       (uint16_t*)out, (uint8_t*)nullptr, (float*)nullptr, 0.0f,
-                       (const uint16_t*)lora_z, (const uint16_t*)lora_b, lora_rank,
-                       order.n_group, order.rotate, a_rows, a_rows != nullptr ? a_total : rows, div.m, div.s);
-  };
+  const V2Args g = {a, a_scale, rows, w, w_scale, 0, experts, n, k, offsets, 0, nullptr, out,
+                    nullptr, nullptr, 0.0f, lora_z, lora_b, lora_rank, a_rows, a_rows_div, partial};
   if (a_rows != nullptr) {
     if (lora_z != nullptr) return 1;  // not a form of this kernel
-    launch(grouped_gemm_v2_kernel<false, false, false, true, false, true>);
-  } else if (lora_z != nullptr) launch(grouped_gemm_v2_kernel<false, false, true, true>);
-  else launch(grouped_gemm_v2_kernel<false, false, false, true>);
-  MI355X_LAUNCH_CHECK();
-  return 0;
+    return launch<false, false, false, true, false, true>(g, stream);
+  }
+  return lora_z != nullptr ? launch<false, false, true, true>(g, stream)
+                           : launch<false, false, false, true>(g, stream);
 }

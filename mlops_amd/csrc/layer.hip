@@ -47,15 +47,17 @@ RouteSpace route_space(void* base, int tokens, int experts, int top_k, int segme
 struct DownSpace {
   uint8_t* q;
   float* scales;
-  void* y;
-  size_t total;
+  void *y, *tail;
+  size_t tail_bytes, total;
 };
-DownSpace down_space(void* base, int rows, int hidden, int inter) {
+DownSpace down_space(void* base, int rows, int hidden, int inter, int experts) {
   Carver c = {(uint8_t*)base, 0};
   DownSpace s;
   s.q = (uint8_t*)c.take((size_t)rows * inter);
   s.scales = (float*)c.take((size_t)rows * (inter / 128) * sizeof(float));
   s.y = c.take((size_t)rows * hidden * 2);
+  s.tail_bytes = mi355x_gemm_tail_workspace_size(rows, experts, hidden, inter);
+  s.tail = s.tail_bytes > 0 ? c.take(s.tail_bytes) : nullptr;
   s.total = c.used;
   return s;
 }
@@ -66,8 +68,8 @@ struct BackwardSpace {
   int32_t* blocks;
   uint8_t *dhq, *dh_t, *ap_t, *gather_t;
   float *dh_scales, *dh_t_scales, *ap_t_scales, *gather_scales, *dscore;
-  void *dx, *swiglu, *router;
-  size_t swiglu_bytes, router_bytes, total;
+  void *dx, *tail, *swiglu, *router;
+  size_t tail_bytes, swiglu_bytes, router_bytes, total;
 };
 BackwardSpace backward_space(void* base, int tokens, int hidden, int inter, int experts, int top_k,
                              int need_w13, int need_w2, int router_kernel) {
@@ -93,6 +95,8 @@ BackwardSpace backward_space(void* base, int tokens, int hidden, int inter, int 
   }
   s.dscore = (float*)c.take(rows * sizeof(float));
   s.dx = c.take(rows * h * 2);
+  s.tail_bytes = mi355x_gemm_tail_workspace_size((int)rows, experts, hidden, 2 * inter);
+  if (s.tail_bytes > 0) s.tail = c.take(s.tail_bytes);
   s.swiglu_bytes = mi355x_swiglu_bwd_quantize_workspace_size((int)rows, inter);
   s.swiglu = c.take(s.swiglu_bytes);
   if (router_kernel) {
@@ -140,8 +144,8 @@ extern "C" int mi355x_moe_route(const float* logits, int tokens, int experts, in
                              s.stats_bytes, stream);
 }
 
-extern "C" size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter) {
-  return down_space(nullptr, rows, hidden, inter).total;
+extern "C" size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter, int experts) {
+  return down_space(nullptr, rows, hidden, inter, experts).total;
 }
 
 extern "C" int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidden, int inter,
@@ -152,18 +156,29 @@ extern "C" int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidde
   MI355X_REQUIRE(tokens >= 0 && top_k > 0 && hidden > 0 && inter > 0 && inter % 128 == 0,
                  "moe_down: bad sizes");
   const int rows = tokens * top_k;
-  const DownSpace s = down_space(workspace, rows, hidden, inter);
+  const DownSpace s = down_space(workspace, rows, hidden, inter, experts);
   MI355X_REQUIRE(workspace_bytes >= s.total, "moe_down: workspace too small");
-  if (row_scaled) {
+  if (row_scaled)
     STEP(mi355x_swiglu_quantize_rows_current_fp8(h13, rows, inter, limit, s.q, s.scales, nullptr,
                                                  stream));
-    STEP(mi355x_gemm_fp8_rowwise(s.q, s.scales, rows, w2, w2_scale, experts, hidden, inter,
-                                 offsets, s.y, stream));
-  } else {
+  else
     STEP(mi355x_swiglu_quantize_fp8(h13, rows, inter, limit, s.q, s.scales, nullptr, stream));
-    STEP(mi355x_gemm_fp8_block(s.q, s.scales, rows, w2, w2_scale, 0, experts, hidden, inter,
-                               offsets, 0, nullptr, s.y, stream));
-  }
+  mi355x_gemm_args g = {};
+  g.a = s.q;
+  g.a_scale = s.scales;
+  g.w = w2;
+  g.w_scale = w2_scale;
+  g.offsets = offsets;
+  g.out = s.y;
+  g.workspace = s.tail;
+  g.workspace_bytes = s.tail_bytes;
+  g.rows = rows;
+  g.a_rows_div = 1;
+  g.experts = experts;
+  g.n = hidden;
+  g.k = inter;
+  g.row_scaled = row_scaled;
+  STEP(mi355x_gemm_fp8(&g, stream));
   return mi355x_unpermute_combine(s.y, slots, weights, residual, tokens, top_k, hidden, out,
                                   stream);
 }
@@ -199,12 +214,23 @@ extern "C" int mi355x_moe_block_bwd(const mi355x_moe_block_bwd_args* a, void* st
                                      padded, a->offsets, a->experts, a->grad_w2,
                                      a->weight_grads_fp32, stream));
   }
-  if (a->w13_kmajor)
-    STEP(mi355x_gemm_fp8_block_kmajor(s.dhq, s.dh_scales, rows, a->w13, a->w13_scale, a->experts,
-                                      h, 2 * i, a->offsets, s.dx, stream));
-  else
-    STEP(mi355x_gemm_fp8_block(s.dhq, s.dh_scales, rows, a->w13, a->w13_scale, 1, a->experts, h,
-                               2 * i, a->offsets, 0, nullptr, s.dx, stream));
+  mi355x_gemm_args g = {};
+  g.a = s.dhq;
+  g.a_scale = s.dh_scales;
+  g.w = a->w13;
+  g.w_scale = a->w13_scale;
+  g.offsets = a->offsets;
+  g.out = s.dx;
+  g.workspace = s.tail;
+  g.workspace_bytes = s.tail_bytes;
+  g.rows = rows;
+  g.a_rows_div = 1;
+  g.experts = a->experts;
+  g.n = h;
+  g.k = 2 * i;
+  g.kmajor = a->w13_kmajor;
+  g.w_scale_t = !a->w13_kmajor;
+  STEP(mi355x_gemm_fp8(&g, stream));
   if (need_w13) {
     if (rows > 0)
       STEP(mi355x_quantize_transpose_fp8(a->x, h, h, a->order, a->top_k, 0, s.blocks, padded,

@@ -593,6 +593,40 @@ def swiglu_bwd_bf16(r, h, weights, order, offsets, *, padded, row_blocks, limit=
 
 
 # ------------------------------------------------------------------- GEMMs
+# mi355x_gemm_args: 11 pointers, the workspace size, eleven ints.
+_GEMM_ARGS = struct.Struct("=12Q11i")
+_TAIL_MIN_K = 4096  # a shorter K is never split (mi355x_gemm_tail_workspace_size is 0)
+
+
+def _run_gemm(name, entry, arguments, a, a_scale, w, w_scale, offsets, out, k, *, a_rows=None,
+              a_total=0, a_rows_div=1, transposed_scale=False, interleave=False,
+              row_scaled=False, kmajor=False, addend=None, z=None, b=None):
+    """One grouped GEMM: ``entry(*arguments)``, or ``mi355x_gemm_fp8`` on the
+    same operands with a workspace where the launch may split its last round
+    of tiles over K."""
+    device = out.device
+    rows, n = out.shape
+    experts = w.shape[0]
+    rank = 0 if z is None else z.shape[1]
+    flops, nbytes = 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n
+    if row_scaled:
+        flops += 2 * rows * n * rank
+    size = 0
+    if k >= _TAIL_MIN_K:
+        size = _native.query("mi355x_gemm_tail_workspace_size", rows, experts, n, k)
+    if size == 0:
+        _timed(name, device, flops, nbytes, entry, *arguments, _stream(device))
+        return out
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    packed = _GEMM_ARGS.pack(
+        *(0 if t is None else t.data_ptr()
+          for t in (a, a_scale, a_rows, w, w_scale, offsets, addend, z, b, out, workspace)),
+        size, rows, a_total, a_rows_div, experts, n, k, int(transposed_scale), int(interleave),
+        int(row_scaled), int(kmajor), rank)
+    _timed(name, device, flops, nbytes, "mi355x_gemm_fp8", packed, _stream(device))
+    return out
+
+
 def gemm(a, a_scale, w, w_scale, offsets, *, transposed_scale=False, interleave=False,
          addend=None, lora=None):
     """Grouped block-FP8 GEMM: bf16 ``[A, N]`` (see the C header for the math).
@@ -612,13 +646,12 @@ def gemm(a, a_scale, w, w_scale, offsets, *, transposed_scale=False, interleave=
         _check(addend, (rows, n), torch.bfloat16, "addend")
     device = _on_gpu(a, a_scale, w, w_scale, offsets, addend)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_block", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_block", _ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale),
-        int(transposed_scale), experts, n, k, _ptr(offsets), int(interleave), _ptr(addend),
-        _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_block", "mi355x_gemm_fp8_block",
+        (_ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale), int(transposed_scale), experts, n,
+         k, _ptr(offsets), int(interleave), _ptr(addend), _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, transposed_scale=transposed_scale,
+        interleave=interleave, addend=addend)
 
 
 def gemm_kmajor(a, a_scale, w, w_scale, offsets):
@@ -637,12 +670,11 @@ def gemm_kmajor(a, a_scale, w, w_scale, offsets):
         raise ValueError("gemm_kmajor: the weight must be contiguous")
     device = _on_gpu(a, a_scale, w, w_scale, offsets)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_block", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_block_kmajor", _ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale),
-        experts, n, k, _ptr(offsets), _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_block", "mi355x_gemm_fp8_block_kmajor",
+        (_ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets),
+         _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, kmajor=True)
 
 
 def quantize_token_rows(x: torch.Tensor):
@@ -689,17 +721,18 @@ def gemm_gathered(a, a_scale, a_rows, w, w_scale, offsets, *, interleave=False, 
         raise ValueError("gemm_gathered: the weight must be contiguous")
     device = _on_gpu(a, a_scale, a_rows, w, w_scale, offsets)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
+    gathered = dict(a_rows=a_rows, a_total=tokens, a_rows_div=int(rows_div))
     if kmajor:
-        _timed("gemm_fp8_block", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-               "mi355x_gemm_fp8_block_kmajor_gathered", _ptr(a), _ptr(a_scale), tokens,
-               _ptr(a_rows), int(rows_div), rows, _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets),
-               _ptr(out), _stream(device))
-    else:
-        _timed("gemm_fp8_block", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-               "mi355x_gemm_fp8_block_gathered", _ptr(a), _ptr(a_scale), tokens, _ptr(a_rows),
-               int(rows_div), rows, _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets), int(interleave),
-               _ptr(out), _stream(device))
-    return out
+        return _run_gemm(
+            "gemm_fp8_block", "mi355x_gemm_fp8_block_kmajor_gathered",
+            (_ptr(a), _ptr(a_scale), tokens, _ptr(a_rows), int(rows_div), rows, _ptr(w),
+             _ptr(w_scale), experts, n, k, _ptr(offsets), _ptr(out)),
+            a, a_scale, w, w_scale, offsets, out, k, kmajor=True, **gathered)
+    return _run_gemm(
+        "gemm_fp8_block", "mi355x_gemm_fp8_block_gathered",
+        (_ptr(a), _ptr(a_scale), tokens, _ptr(a_rows), int(rows_div), rows, _ptr(w),
+         _ptr(w_scale), experts, n, k, _ptr(offsets), int(interleave), _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, interleave=interleave, **gathered)
 
 
 def rank_product(a, bt, offsets, *, splits=None):
@@ -800,13 +833,12 @@ def _gemm_lora(a, a_scale, w, w_scale, offsets, transposed_scale, interleave, z,
     _check(b, (experts, n, rank), torch.bfloat16, "LoRA b")
     device = _on_gpu(a, a_scale, w, w_scale, offsets, z, b)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_block", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_block_lora", _ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale),
-        int(transposed_scale), experts, n, k, _ptr(offsets), int(interleave), _ptr(z), _ptr(b),
-        rank, _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_block", "mi355x_gemm_fp8_block_lora",
+        (_ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale), int(transposed_scale), experts, n,
+         k, _ptr(offsets), int(interleave), _ptr(z), _ptr(b), rank, _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, transposed_scale=transposed_scale,
+        interleave=interleave, z=z, b=b)
 
 
 def gemm_swiglu(a, a_scale, w, w_scale, offsets, *, limit=None, addend=None):
@@ -819,6 +851,10 @@ def gemm_swiglu(a, a_scale, w, w_scale, offsets, *, limit=None, addend=None):
         raise ValueError(f"weight K {kw} != activation K {k}")
     _check(a_scale, (k // 128, rows), torch.float32, "activation scales")
     device = _on_gpu(a, a_scale, w, w_scale, offsets, addend)
+    if k >= _TAIL_MIN_K and _native.query("mi355x_gemm_tail_workspace_size", rows, experts, n, k):
+        # The GEMM whose last round may be split, then the SwiGLU pass: h as gemm() gives it.
+        h = gemm(a, a_scale, w, w_scale, offsets, interleave=True, addend=addend)
+        return (h, *swiglu_quantize(h, limit=limit))
     h = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
     act = torch.empty((rows, n // 2), dtype=FP8, device=device)
     act_scales = torch.empty((n // 256, rows), dtype=torch.float32, device=device)
@@ -924,12 +960,11 @@ def gemm_rowwise(a, a_scale, w, w_scale, offsets, *, lora=None):
     _check(offsets, (experts + 1,), torch.int32, "offsets")
     device = _on_gpu(a, a_scale, w, w_scale, offsets)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_rowwise", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_rowwise", _ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale),
-        experts, n, k, _ptr(offsets), _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_rowwise", "mi355x_gemm_fp8_rowwise",
+        (_ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets),
+         _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, row_scaled=True)
 
 
 def gemm_rowwise_gathered(a, a_scale, a_rows, w, w_scale, offsets, *, rows_div=1):
@@ -948,13 +983,12 @@ def gemm_rowwise_gathered(a, a_scale, a_rows, w, w_scale, offsets, *, rows_div=1
     _check(offsets, (experts + 1,), torch.int32, "offsets")
     device = _on_gpu(a, a_scale, a_rows, w, w_scale, offsets)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_rowwise", device, 2 * rows * n * k, rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_rowwise_gathered", _ptr(a), _ptr(a_scale), tokens, _ptr(a_rows),
-        int(rows_div), rows,
-        _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets), _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_rowwise", "mi355x_gemm_fp8_rowwise_gathered",
+        (_ptr(a), _ptr(a_scale), tokens, _ptr(a_rows), int(rows_div), rows, _ptr(w),
+         _ptr(w_scale), experts, n, k, _ptr(offsets), _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, row_scaled=True, a_rows=a_rows, a_total=tokens,
+        a_rows_div=int(rows_div))
 
 
 def _gemm_rowwise_lora(a, a_scale, w, w_scale, offsets, z, b):
@@ -972,13 +1006,11 @@ def _gemm_rowwise_lora(a, a_scale, w, w_scale, offsets, z, b):
         raise ValueError("lora factors must be contiguous")
     device = _on_gpu(a, a_scale, w, w_scale, offsets, z, b)
     out = torch.empty((rows, n), dtype=torch.bfloat16, device=device)
-    _timed(
-        "gemm_fp8_rowwise", device, 2 * rows * n * (k + rank),
-        rows * k + experts * n * k + 2 * rows * n,
-        "mi355x_gemm_fp8_rowwise_lora", _ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale),
-        experts, n, k, _ptr(offsets), _ptr(z), _ptr(b), rank, _ptr(out), _stream(device),
-    )
-    return out
+    return _run_gemm(
+        "gemm_fp8_rowwise", "mi355x_gemm_fp8_rowwise_lora",
+        (_ptr(a), _ptr(a_scale), rows, _ptr(w), _ptr(w_scale), experts, n, k, _ptr(offsets),
+         _ptr(z), _ptr(b), rank, _ptr(out)),
+        a, a_scale, w, w_scale, offsets, out, k, row_scaled=True, z=z, b=b)
 
 
 def wgrad(p, p_scale, q, q_scale, offsets, *, out_dtype=torch.bfloat16, rows=None):
@@ -1082,7 +1114,7 @@ def moe_down(h13, w2, w2_scale, offsets, slots, weights, residual, limit=None, *
     _check(residual, (tokens, hidden), torch.bfloat16, "residual")
     device = _on_gpu(h13, w2, w2_scale, offsets, slots, weights, residual)
     out = torch.empty_like(residual)
-    size = _native.query("mi355x_moe_down_workspace_size", rows, hidden, inter)
+    size = _native.query("mi355x_moe_down_workspace_size", rows, hidden, inter, experts)
     work = torch.empty(size, dtype=torch.uint8, device=device)
     _native.call("mi355x_moe_down", _ptr(h13), tokens, top_k, hidden, inter, _limit(limit),
                  int(row_scaled), _ptr(w2), _ptr(w2_scale), experts, _ptr(offsets), _ptr(slots),

@@ -486,6 +486,81 @@ def test_grouped_gemm_forms_at_every_tile_size(device, counts, n, k):
     assert worst_cell_rel(out.cpu(), want, offsets.tolist()) < 4e-3
 
 
+@pytest.mark.parametrize("counts,n,k", [
+    ([300, 511, 0, 900, 130], 8192, 4096),  # a full round, then 4 tiles an XCD in 4 parts
+    ([500, 400, 300, 500], 4096, 8192),  # fewer tiles than CUs: 16 an XCD in 2 parts
+    ([1000, 900, 800, 700, 600, 620], 4096, 8192),  # a full round, then 10 an XCD in 3
+])
+def test_grouped_gemm_last_round_split_over_k(device, monkeypatch, counts, n, k):
+    """Every form whose last round of tiles is split over K against the whole
+    tiles' result, and the plain ones against the fp64 product. Both results
+    are one bf16 rounding (2^-9 of each element) of fp32 sums that agree to
+    1e-6, so they differ by at most 2 * 2^-9 < 4e-3 of a cell's norm."""
+    g = torch.Generator(device=device).manual_seed(n + k)
+    offsets = _ragged(counts).to(device)
+    bounds = offsets.tolist()
+    rows, experts, tokens = bounds[-1], len(counts), 301
+    assert K._native.query("mi355x_gemm_tail_workspace_size", rows, experts, n, k) > 0
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g, device=device) * std).to(torch.bfloat16)
+
+    def product(a, w):
+        out = torch.empty(rows, n, dtype=torch.float64, device=device)
+        for e, (lo, hi) in enumerate(zip(bounds, bounds[1:])):
+            out[lo:hi] = a(lo, hi) @ w(e).t()
+        return out
+
+    slots = torch.randint(0, 3 * tokens, (rows,), generator=g, device=device).to(torch.int32)
+    x = normal(tokens, k)
+    routed = x[(slots // 3).long()]
+    w = normal(experts, n, k, std=0.02)
+    xq, xs = K.quantize_rows(routed)
+    tq, ts = K.quantize_token_rows(x)
+    wq, ws = K.quantize_weight_blocks(w)
+    kq, ks = K.quantize_weight_blocks(w.transpose(1, 2).contiguous())
+    kt = K.transpose_fp8(kq)
+    rq, _, rs, _ = K.quantize_weights_current(w)
+    cq, cs = K.quantize_rows_current(routed)
+    ctq, cts = K.quantize_rows_current(x)
+    c, z, b = normal(rows, n), normal(rows, 16, std=0.5), normal(experts, n, 16, std=0.1)
+    forms = dict(
+        plain=lambda: K.gemm(xq, xs, wq, ws, offsets),
+        gathered=lambda: K.gemm_gathered(tq, ts, slots, wq, ws, offsets, rows_div=3),
+        interleaved=lambda: K.gemm(xq, xs, wq, ws, offsets, interleave=True),
+        swiglu=lambda: K.gemm_swiglu(xq, xs, wq, ws, offsets)[0],
+        addend=lambda: K.gemm(xq, xs, wq, ws, offsets, addend=c),
+        rank=lambda: K.gemm(xq, xs, wq, ws, offsets, lora=(z, b)),
+        transposed=lambda: K.gemm(xq, xs, kt, ks, offsets, transposed_scale=True),
+        kmajor=lambda: K.gemm_kmajor(xq, xs, kq, ks, offsets),
+        kmajor_gathered=lambda: K.gemm_gathered(tq, ts, slots, kq, ks, offsets, kmajor=True,
+                                                rows_div=3),
+        rows=lambda: K.gemm_rowwise(cq, cs, rq, rs, offsets),
+        rows_gathered=lambda: K.gemm_rowwise_gathered(ctq, cts, slots, rq, rs, offsets,
+                                                      rows_div=3),
+        rows_rank=lambda: K.gemm_rowwise(cq, cs, rq, rs, offsets, lora=(z, b)),
+    )
+    split = {name: form() for name, form in forms.items()}
+    for name, form in forms.items():
+        assert torch.equal(split[name], form()), name  # the parts are added in a fixed order
+    for name, same in (("plain", "gathered"), ("interleaved", "swiglu"),
+                       ("transposed", "kmajor"), ("kmajor", "kmajor_gathered"),
+                       ("rows", "rows_gathered")):
+        assert torch.equal(split[name], split[same]), same
+    monkeypatch.setattr(K, "_TAIL_MIN_K", 1 << 30)
+    for name, form in forms.items():
+        whole = form()
+        if not name.startswith("rows"):  # (unscaled e4m3 products add up exactly)
+            assert not torch.equal(split[name], whole), name  # the split did run
+        assert worst_cell_rel(split[name], whole, bounds) < 4e-3, name
+    xd = xq.double() * xs.t().double().repeat_interleave(128, 1)
+    wd = lambda e: wq[e].double() * ws[e].double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    assert worst_cell_rel(split["plain"], product(lambda lo, hi: xd[lo:hi], wd), bounds) < 4e-3
+    cd = cq.double() * cs.double()[:, None]
+    rd = lambda e: rq[e].double() * rs[e].double()[:, None]
+    assert worst_cell_rel(split["rows"], product(lambda lo, hi: cd[lo:hi], rd), bounds) < 4e-3
+
+
 
 @pytest.mark.parametrize("tokens,top_k,experts,k,n,form", [
     (2000, 4, 16, 512, 512, "up"),           # gate/up interleave, partial row tiles

@@ -548,6 +548,7 @@ def test_gathered_token_rows_equal_permuted_copy_in_the_layer(device, monkeypatc
 
 
 @pytest.mark.parametrize("precision,tokens,experts,top_k,inter,mode", [
+    ("fp8_block", 768, 4, 2, 6144, "topk_then_softmax"),     # last rounds split over K
     ("fp8_block", 1, 8, 2, 256, "topk_then_softmax"),        # the smallest call
     ("fp8_block", 97, 64, 8, 256, "softmax_then_topk"),      # router gradient on its kernel
     ("fp8_block", 130, 8, 3, 384, "sigmoid_noaux_tc"),       # w2's transposed copy, sequences
@@ -559,9 +560,14 @@ def test_launch_sequences_equal_single_kernel_calls(device, precision, tokens, e
                                                     inter, mode):
     """The layer's native launch sequences give the bytes of the same kernels
     called one at a time (as they are while a launch timer is installed)."""
-    x, res, wr, w13, w2, dy = _inputs(device, tokens=tokens, hidden=256, experts=experts,
+    hidden = 4096 if inter == 6144 else 256
+    x, res, wr, w13, w2, dy = _inputs(device, tokens=tokens, hidden=hidden, experts=experts,
                                       inter=inter, seed=13)
     lengths = (tokens // 2, tokens - tokens // 2) if tokens == 130 else None
+    if hidden == 4096:  # the down projection and the input gradient
+        for k in (inter, 2 * inter):
+            assert K._native.query("mi355x_gemm_tail_workspace_size", tokens * top_k, experts,
+                                   hidden, k) > 0
 
     def run():
         leaves = [t.clone().requires_grad_(True) for t in (x, wr, w13, w2)]
