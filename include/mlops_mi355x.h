@@ -541,6 +541,26 @@ int mi355x_moe_route(const float* logits, int tokens, int experts, int top_k, in
                      int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
                      float* aux, float* prob_sum, void* workspace, size_t workspace_bytes,
                      void* stream);
+/* mi355x_moe_route from the token rows: logits [T, E] of x [T, width] (bf16)
+ * through the router weight [E, width] (bf16, or fp32 rounded to bf16), bf16
+ * products and fp32 sums, then the routing (kernels/router.py:54-74). With
+ * `quantize` the token rows too: q e4m3 [T, width] and scales [T, width/128]
+ * (as mi355x_quantize_token_rows_fp8) or [T] (as
+ * mi355x_quantize_rows_current_fp8). At most 64 tokens, 128 experts, top_k 16,
+ * no group limit, one sequence, width a multiple of 128, operands 16-byte
+ * aligned; the workspace size is 0 outside that range. */
+#define MI355X_ROUTE_QUANTIZE_NONE 0
+#define MI355X_ROUTE_QUANTIZE_BLOCKS 1
+#define MI355X_ROUTE_QUANTIZE_ROWS 2
+size_t mi355x_moe_route_tokens_workspace_size(int tokens, int experts, int top_k, int mode,
+                                              int n_group, int topk_group, int width);
+int mi355x_moe_route_tokens(const void* x, const void* weight, int weight_fp32, int tokens,
+                            int experts, int width, int quantize, uint8_t* q, float* scales,
+                            int top_k, int mode, const float* bias, int n_group, int topk_group,
+                            float routed_scaling, const int32_t* forced_ids, float* logits,
+                            float* weights, int32_t* ids, int64_t* counts, int32_t* offsets,
+                            int32_t* order, int32_t* slots, float* aux, float* prob_sum,
+                            void* workspace, size_t workspace_bytes, void* stream);
 size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter, int experts);
 int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidden, int inter, float limit,
                     int row_scaled, const uint8_t* w2, const float* w2_scale, int experts,

@@ -101,6 +101,9 @@ SIGNATURES = {
     "mi355x_moe_route_workspace_size": (_S, [_I, _I, _I, _I, _I]),
     "mi355x_moe_route": (_I, [_P, _I, _I, _I, _I, _P, _I, _I, _F, _P, _I, _P, _P, _I, _P, _P, _P,
                               _P, _P, _P, _P, _P, _P, _S, _P]),
+    "mi355x_moe_route_tokens_workspace_size": (_S, [_I] * 7),
+    "mi355x_moe_route_tokens": (_I, [_P, _P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _P, _I, _I, _F,
+                                     _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _S, _P]),
     "mi355x_moe_down_workspace_size": (_S, [_I] * 4),
     "mi355x_moe_down": (_I, [_P, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _S,
                              _P]),

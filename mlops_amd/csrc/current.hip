@@ -8,16 +8,10 @@
 // The kernels are HBM-bound. A row kernel reads its row twice, once for the
 // maximum and once to quantize it; the second read hits the caches. Widths
 // reach 28672 (Mixtral's gate/up rows), too wide to hold in registers.
-#include "common.h"
+#include "row_quant.h"
 
 namespace {
 
-template <typename T>
-__device__ __forceinline__ void load8(const T* p, float* v);
-template <>
-__device__ __forceinline__ void load8<uint16_t>(const uint16_t* p, float* v) {
-  load_bf16x8(p, v);
-}
 // Weights: read once per pass, through non-temporal loads.
 template <typename T>
 __device__ __forceinline__ void load8_once(const T* p, float* v) { load8(p, v); }
@@ -25,13 +19,6 @@ template <>
 __device__ __forceinline__ void load8_once<uint16_t>(const uint16_t* p, float* v) {
   unpack_bf16x8(load_stream(p), v);
 }
-template <>
-__device__ __forceinline__ void load8<float>(const float* p, float* v) {
-  const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-
 // Source row of stored row r: a gathered routed row (gather[r] / div, the
 // token of a sorted assignment), a weight row in gate/up-adjacent order
 // (stored row 2j of an expert = gate row j, 2j + 1 = up row j; interleave =
@@ -56,27 +43,7 @@ __global__ void __launch_bounds__(256) rows_current_kernel(
   const int r = blockIdx.x * 4 + wave;
   if (r >= rows) return;
   const T* src = x + source_row(r, gather, div, interleave) * pitch;
-  float amax = 0.0f;
-  for (int col = lane * 8; col < width; col += 512) {
-    float v[8];
-    load8(src + col, v);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-  }
-  amax = group_amax<64>(amax);
-  const float s = fmaxf(amax * kInv448, kMinScale);
-  uint8_t* dst = q + (size_t)r * width;
-  // Four chunks' loads before their stores: loads and stores complete in
-  // order, so a load issued after a store would wait for it.
-  for (int col0 = lane * 8; col0 < width; col0 += 4 * 512) {
-    float v[4][8];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (col0 + c * 512 < width) load8(src + col0 + c * 512, v[c]);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (col0 + c * 512 < width) *(uint2*)(dst + col0 + c * 512) = quant8(v[c], s);
-  }
+  const float s = quantize_row_current(src, width, q + (size_t)r * width);
   if (lane == 0) scales[r] = s;
 }
 

@@ -8,11 +8,18 @@
 #include "common.h"
 
 // router.hip: the routing of at most 64 tokens; returns 1 outside its range.
-int mi355x_route_small(const float* logits, int tokens, int experts, int top_k, int mode,
-                       const float* bias, int n_group, int topk_group, float routed_scaling,
-                       const int32_t* forced_ids, int segments, float* weights, int32_t* ids,
-                       int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
-                       float* aux, float* prob_sum, void* stream);
+bool mi355x_route_small_serves(int tokens, int experts, int top_k, int mode, int n_group,
+                               int topk_group, int segments);
+int mi355x_route_small(float* logits, const float* partial, int parts, int tokens, int experts,
+                       int top_k, int mode, const float* bias, int n_group, int topk_group,
+                       float routed_scaling, const int32_t* forced_ids, int segments,
+                       float* weights, int32_t* ids, int64_t* counts, int32_t* offsets,
+                       int32_t* order, int32_t* slots, float* aux, float* prob_sum, void* stream);
+// router_logits.hip: its logits in parts, and the quantized token rows.
+int mi355x_router_logits_parts(int width);
+int mi355x_router_logits_launch(const void* x, const void* weight, int weight_fp32, int tokens,
+                                int experts, int width, float* partial, int pitch, int quantize,
+                                uint8_t* q, float* scales, void* stream);
 
 namespace {
 
@@ -131,9 +138,10 @@ extern "C" int mi355x_moe_route(const float* logits, int tokens, int experts, in
   MI355X_REQUIRE(tokens >= 0 && experts > 0 && top_k > 0, "moe_route: bad sizes");
   const RouteSpace s = route_space(workspace, tokens, experts, top_k, segments, nchunks);
   MI355X_REQUIRE(workspace_bytes >= s.total, "moe_route: workspace too small");
-  const int small = mi355x_route_small(logits, tokens, experts, top_k, mode, bias, n_group,
-                                       topk_group, routed_scaling, forced_ids, segments, weights,
-                                       ids, counts, offsets, order, slots, aux, prob_sum, stream);
+  const int small = mi355x_route_small((float*)logits, nullptr, 0, tokens, experts, top_k, mode,
+                                       bias, n_group, topk_group, routed_scaling, forced_ids,
+                                       segments, weights, ids, counts, offsets, order, slots, aux,
+                                       prob_sum, stream);
   if (small <= 0) return small;
   STEP(mi355x_router_topk(logits, tokens, experts, top_k, mode, bias, n_group, topk_group,
                           routed_scaling, forced_ids, weights, ids, stream));
@@ -142,6 +150,45 @@ extern "C" int mi355x_moe_route(const float* logits, int tokens, int experts, in
   return mi355x_router_stats(logits, ids, tokens, experts, top_k, mode, segments, seg_offsets,
                              chunk_table, nchunks, aux, prob_sum, s.seg_counts, s.stats,
                              s.stats_bytes, stream);
+}
+
+extern "C" size_t mi355x_moe_route_tokens_workspace_size(int tokens, int experts, int top_k,
+                                                         int mode, int n_group, int topk_group,
+                                                         int width) {
+  if (width <= 0 || width % 128 != 0 || experts <= 0 || top_k <= 0 ||
+      !mi355x_route_small_serves(tokens, experts, top_k, mode, n_group, topk_group, 1))
+    return 0;
+  const size_t pitch = ((size_t)tokens * experts + 3) / 4 * 4;
+  return mi355x_router_logits_parts(width) * pitch * sizeof(float);
+}
+
+extern "C" int mi355x_moe_route_tokens(const void* x, const void* weight, int weight_fp32,
+                                       int tokens, int experts, int width, int quantize,
+                                       uint8_t* q, float* scales, int top_k, int mode,
+                                       const float* bias, int n_group, int topk_group,
+                                       float routed_scaling, const int32_t* forced_ids,
+                                       float* logits, float* weights, int32_t* ids,
+                                       int64_t* counts, int32_t* offsets, int32_t* order,
+                                       int32_t* slots, float* aux, float* prob_sum,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+  const size_t need = mi355x_moe_route_tokens_workspace_size(tokens, experts, top_k, mode, n_group,
+                                                             topk_group, width);
+  MI355X_REQUIRE(need > 0, "moe_route_tokens: outside the range of the fused routing");
+  MI355X_REQUIRE(workspace_bytes >= need, "moe_route_tokens: workspace too small");
+  MI355X_REQUIRE(quantize >= MI355X_ROUTE_QUANTIZE_NONE && quantize <= MI355X_ROUTE_QUANTIZE_ROWS,
+                 "moe_route_tokens: unknown quantization %d", quantize);
+  MI355X_REQUIRE(quantize == MI355X_ROUTE_QUANTIZE_NONE || (q != nullptr && scales != nullptr),
+                 "moe_route_tokens: the quantized rows need q and scales");
+  MI355X_REQUIRE((((uintptr_t)x | (uintptr_t)weight) & 15) == 0,
+                 "moe_route_tokens: operands must be 16-byte aligned");
+  MI355X_REQUIRE(((uintptr_t)workspace & 15) == 0,
+                 "moe_route_tokens: the workspace must be 16-byte aligned");
+  float* partial = (float*)workspace;
+  STEP(mi355x_router_logits_launch(x, weight, weight_fp32, tokens, experts, width, partial,
+                                   (tokens * experts + 3) / 4 * 4, quantize, q, scales, stream));
+  return mi355x_route_small(logits, partial, mi355x_router_logits_parts(width), tokens, experts,
+                            top_k, mode, bias, n_group, topk_group, routed_scaling, forced_ids, 1,
+                            weights, ids, counts, offsets, order, slots, aux, prob_sum, stream);
 }
 
 extern "C" size_t mi355x_moe_down_workspace_size(int rows, int hidden, int inter, int experts) {

@@ -2,7 +2,7 @@
 // backward row pass. All of them are HBM-bound byte/element work: each reads
 // its source once with 16-byte vector loads and writes e4m3 with 8- or
 // 16-byte stores; 128-element scale groups are formed by 16-lane shuffles.
-#include "common.h"
+#include "row_quant.h"
 
 namespace {
 
@@ -119,43 +119,12 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(const uint16_t* __re
   const int r = blockIdx.x * 4 + wave;
   if (r >= rows) return;
   const uint16_t* src = x + (size_t)r * pitch;
-  // Up to four 512-column chunks' loads are issued before any of their
-  // stores: loads and stores share one completion counter, so a load issued
-  // after a store would wait for it.
-  constexpr int kChunks = 4;
   if (!gate_up) {
-    for (int base0 = 0; base0 < width; base0 += 512 * kChunks) {
-      uint4 raw[kChunks];
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) {
-        const int col = base0 + c * 512 + lane * 8;
-        raw[c] = col < width ? *(const uint4*)(src + col) : make_uint4(0, 0, 0, 0);
-      }
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) {
-        if (base0 + c * 512 >= width) break;  // uniform over the wave
-        const int col = base0 + c * 512 + lane * 8;
-        float v[8];
-        unpack_bf16x8(raw[c], v);
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        amax = group_amax<16>(amax);
-        const float s = fmaxf(amax * kInv448, kMinScale);
-        const uint2 packed = quant8(v, s);
-        if (col < width) {
-          store_stream8(q + (size_t)r * width + col, packed);
-          if ((lane & 15) == 0) {
-            const size_t si = row_scales ? (size_t)r * (width >> 7) + (col >> 7)
-                                         : (size_t)(col >> 7) * rows + r;
-            scales[si] = s;
-          }
-        }
-      }
-    }
+    quantize_row_blocks(src, r, rows, width, row_scales, q, scales);
     return;
   }
   const int half = width / 2;
+  constexpr int kChunks = 4;  // loads before stores, as in quantize_row_blocks
   for (int base0 = 0; base0 < half; base0 += 512 * kChunks) {
     uint4 ra[kChunks], rb[kChunks];
 #pragma unroll

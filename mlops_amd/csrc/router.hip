@@ -589,8 +589,9 @@ __global__ void __launch_bounds__(kFinishThreads) router_stats_finish_kernel(
 constexpr int kSmallTokens = kStatsChunk, kSmallThreads = 16 * kSmallTokens;
 template <int PL>
 __global__ void __launch_bounds__(kSmallThreads) route_small_kernel(
-    const float* __restrict__ logits, int tokens, int experts, int top_k, int mode,
-    const float* __restrict__ bias, float routed_scaling, const int32_t* __restrict__ forced,
+    float* logits, const float* __restrict__ partial, int parts, int tokens, int experts,
+    int top_k, int mode, const float* __restrict__ bias, float routed_scaling,
+    const int32_t* __restrict__ forced,
     float* __restrict__ weights, int32_t* __restrict__ ids, int64_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ order, int32_t* __restrict__ slots,
     float* __restrict__ aux, float* __restrict__ prob_sum) {
@@ -604,6 +605,22 @@ __global__ void __launch_bounds__(kSmallThreads) route_small_kernel(
   if (tid < kRowExperts) count[tid] = 0;
   for (int j = tid; j < kWavesHere * kRowExperts / 4; j += kSmallThreads)
     ((uint32_t*)wave_count)[j] = 0;
+  // Logits still in (up to four) parts over K: added in order, four at a time.
+  if (parts > 0) {
+    const int pairs = tokens * experts, pitch = (pairs + 3) & ~3;
+    for (int i = 4 * tid; i < pairs; i += 4 * kSmallThreads) {
+      v4f part[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) part[p] = *(const v4f*)(partial + min(p, parts - 1) * pitch + i);
+      v4f total = part[0];
+#pragma unroll
+      for (int p = 1; p < 4; ++p)
+        if (p < parts) total += part[p];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j < pairs) logits[i + j] = total[j];
+    }
+  }
   __syncthreads();
   if (token < tokens) {
     float w;
@@ -937,21 +954,29 @@ extern "C" int mi355x_router_topk(const float* logits, int tokens, int experts, 
   return MI355X_OK;
 }
 
-// Top-k, plan and statistics in one launch; returns 1 outside its range.
-int mi355x_route_small(const float* logits, int tokens, int experts, int top_k, int mode,
-                       const float* bias, int n_group, int topk_group, float routed_scaling,
-                       const int32_t* forced_ids, int segments, float* weights, int32_t* ids,
-                       int64_t* counts, int32_t* offsets, int32_t* order, int32_t* slots,
-                       float* aux, float* prob_sum, void* stream) {
-  if (tokens < 1 || tokens > kSmallTokens || segments != 1 || experts > kRowExperts ||
-      top_k > kRowTopK || (mode == MI355X_ROUTE_SIGMOID_NOAUX_TC && topk_group < n_group))
+bool mi355x_route_small_serves(int tokens, int experts, int top_k, int mode, int n_group,
+                               int topk_group, int segments) {
+  return tokens >= 1 && tokens <= kSmallTokens && segments == 1 && experts <= kRowExperts &&
+         top_k <= kRowTopK && !(mode == MI355X_ROUTE_SIGMOID_NOAUX_TC && topk_group < n_group);
+}
+
+// Top-k, plan and statistics in one launch; returns 1 outside its range. With
+// parts > 0 (at most 4) the logits are formed first, from partial [parts][pitch],
+// pitch = tokens * experts rounded up to 4, 16-byte aligned.
+int mi355x_route_small(float* logits, const float* partial, int parts, int tokens, int experts,
+                       int top_k, int mode, const float* bias, int n_group, int topk_group,
+                       float routed_scaling, const int32_t* forced_ids, int segments,
+                       float* weights, int32_t* ids, int64_t* counts, int32_t* offsets,
+                       int32_t* order, int32_t* slots, float* aux, float* prob_sum,
+                       void* stream) {
+  if (!mi355x_route_small_serves(tokens, experts, top_k, mode, n_group, topk_group, segments))
     return 1;
   const int c = topk_checks(tokens, experts, top_k, mode, n_group, topk_group);
   if (c != MI355X_OK) return c;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(1), dim3(kSmallThreads), 0, (hipStream_t)stream, logits,
-                       tokens, experts, top_k, mode, bias, routed_scaling, forced_ids, weights,
-                       ids, counts, offsets, order, slots, aux, prob_sum);
+                       partial, parts, tokens, experts, top_k, mode, bias, routed_scaling,
+                       forced_ids, weights, ids, counts, offsets, order, slots, aux, prob_sum);
   };
   const int need = (experts + 15) / 16;
   if (need <= 1) launch(route_small_kernel<1>);

@@ -1087,6 +1087,65 @@ def route(logits, top_k: int, mode: str, lengths: Sequence[int], *, bias=None, n
     return weights, ids, counts, offsets, order, slots, aux, prob_sum
 
 
+_ROUTE_TOKENS = 64
+_ROUTE_QUANTIZE = {None: 0, "blocks": 1, "rows": 2}
+
+
+def route_tokens(x, weight, top_k: int, mode: str, lengths: Sequence[int], *, bias=None,
+                 n_group=1, topk_group=1, routed_scaling=1.0, forced_ids=None, quantize=None):
+    """``(logits, rows, (weights, ids, counts, offsets, order, slots, aux,
+    prob_sum))`` of a few token rows ``x bf16 [T, H]`` through a bf16 or fp32
+    router ``weight [E, H]``: the router GEMM and :func:`route` in two launches
+    (``mi355x_moe_route_tokens``), or None outside their range. ``rows``: with
+    ``quantize="blocks"`` :func:`quantize_token_rows`'s pair, with ``"rows"``
+    :func:`quantize_rows_current`'s."""
+    tokens, width = x.shape
+    if tokens > _ROUTE_TOKENS or len(lengths) > 1 or mode not in ROUTING_MODES:
+        return None
+    if (x.dtype != torch.bfloat16 or weight.dtype not in (torch.float32, torch.bfloat16)
+            or weight.device != x.device or not x.is_contiguous() or not weight.is_contiguous()
+            or (x.data_ptr() | weight.data_ptr()) & 15):
+        return None
+    experts = weight.shape[0]
+    size = _native.query("mi355x_moe_route_tokens_workspace_size", tokens, experts, top_k,
+                         ROUTING_MODES[mode], n_group, topk_group, width)
+    if size == 0:
+        return None
+    if bias is not None:
+        bias = bias.float().contiguous()
+        if bias.shape != (experts,):
+            raise ValueError("router bias must be [experts]")
+    if forced_ids is not None:
+        forced_ids = forced_ids.to(device=x.device, dtype=torch.int32).contiguous()
+        _check(forced_ids, (tokens, top_k), torch.int32, "forced_ids")
+    device = _on_gpu(x, weight, bias, forced_ids)
+    rows = None
+    if quantize is not None:
+        rows = (torch.empty((tokens, width), dtype=FP8, device=device),
+                torch.empty((tokens, width // 128) if quantize == "blocks" else tokens,
+                            dtype=torch.float32, device=device))
+    q, scales = rows or (None, None)
+    logits = torch.empty((tokens, experts), dtype=torch.float32, device=device)
+    weights = torch.empty((tokens, top_k), dtype=torch.float32, device=device)
+    ids = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
+    counts = torch.empty(experts, dtype=torch.int64, device=device)
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device=device)
+    order = torch.empty(tokens * top_k, dtype=torch.int32, device=device)
+    slots = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
+    aux = torch.empty((), dtype=torch.float32, device=device)
+    prob_sum = torch.empty(experts, dtype=torch.float32, device=device)
+    work = torch.empty(size, dtype=torch.uint8, device=device)
+    _timed("route_tokens", device, 2 * tokens * experts * width,
+           weight.element_size() * experts * width + 2 * tokens * width,
+           "mi355x_moe_route_tokens", _ptr(x), _ptr(weight), int(weight.dtype == torch.float32),
+           tokens, experts, width, _ROUTE_QUANTIZE[quantize], _ptr(q), _ptr(scales), top_k,
+           ROUTING_MODES[mode], _ptr(bias), n_group, topk_group, routed_scaling,
+           _ptr(forced_ids), _ptr(logits), _ptr(weights), _ptr(ids), _ptr(counts), _ptr(offsets),
+           _ptr(order), _ptr(slots), _ptr(aux), _ptr(prob_sum), _ptr(work), size,
+           _stream(device))
+    return logits, rows, (weights, ids, counts, offsets, order, slots, aux, prob_sum)
+
+
 def moe_down(h13, w2, w2_scale, offsets, slots, weights, residual, limit=None, *,
              row_scaled=False):
     """``residual + sum_j weights[t, j] y[slots[t, j]]`` for the down projection

@@ -162,18 +162,25 @@ def forward_routed(
     with torch.no_grad():
         x = h2.reshape(rows, width).contiguous()
         base = residual.reshape(rows, width).contiguous()
-        logits = router.router_logits(x, router_weight)
         forced = next_override(rows, experts, top_k, x.device) if use_routing_override else None
         bias = None if router_bias is None or router_bias.numel() == 0 else router_bias
-        weights, ids, counts, offsets, order, slots, aux, probability_sum = kernels.route(
-            logits, int(top_k), routing_mode, lengths, bias=bias, n_group=int(n_group),
-            topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced,
-        )
+        options = dict(bias=bias, n_group=int(n_group), topk_group=int(topk_group),
+                       routed_scaling=float(routed_scaling), forced_ids=forced)
+        gathered = _reads_token_rows(int(top_k), w13_data.shape[1])
+        fused_routing = kernels.route_tokens(
+            x, router_weight, int(top_k), routing_mode, lengths,
+            quantize="blocks" if gathered else None, **options)
+        if fused_routing is not None:
+            logits, quantized, routing = fused_routing
+        else:
+            logits, quantized = router.router_logits(x, router_weight), None
+            routing = kernels.route(logits, int(top_k), routing_mode, lengths, **options)
+        weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
         # GEMM, then the SwiGLU pass: measured faster than the fused epilogue
         # of mi355x_gemm_fp8_block_swiglu, whose activation math runs while
         # every wave of the CU is in the epilogue (no MFMA work to hide it).
         h13 = routed_rows_gemm(x, slots, order, int(top_k), (w13_data, w13_scale), offsets,
-                               interleave=True)
+                               interleave=True, quantized=quantized)
         output = kernels.moe_down(h13, w2_data, w2_scale, offsets, slots, weights, base,
                                   swiglu_limit)
     return (output.reshape(h2.shape), aux, counts, probability_sum, logits, weights, ids, order,
@@ -345,18 +352,24 @@ def _split(w13, w2, weight_components):
 GATHER_MIN_TOP_K = 4
 
 
+def _reads_token_rows(top_k: int, n: int) -> bool:
+    """Whether :func:`routed_rows_gemm` reads the token rows, quantized once,
+    rather than their permuted copy."""
+    return top_k >= GATHER_MIN_TOP_K and n % 256 == 0
+
+
 def routed_rows_gemm(x, slots, order, top_k, weight, offsets, *, interleave=False,
-                     input_gradient=False):
+                     input_gradient=False, quantized=None):
     """The GEMM on the routed rows of token rows ``x [T, K]`` (bf16): the
     projection ``rows @ W[e]^T`` (``weight = (data [E, N, K], scale)``), or
     with ``input_gradient`` the input gradient ``rows @ W[e]`` as
     :func:`input_gradient_gemm` does it. Bitwise the same whichever way the
-    rows are read."""
+    rows are read. ``quantized``: the token rows' quantization, where it is at hand."""
     data, scale = weight[0], weight[1]
     n = data.shape[2] if input_gradient else data.shape[1]
     kmajor = input_gradient and len(weight) == 2
-    if top_k >= GATHER_MIN_TOP_K and n % 256 == 0 and (kmajor or not input_gradient):
-        tq, ts = kernels.quantize_token_rows(x)
+    if _reads_token_rows(top_k, n) and (kmajor or not input_gradient):
+        tq, ts = kernels.quantize_token_rows(x) if quantized is None else quantized
         # Routed row r reads token order[r] // top_k, divided in the kernel.
         return kernels.gemm_gathered(tq, ts, order, data, scale, offsets, interleave=interleave,
                                      kmajor=kmajor, rows_div=top_k)

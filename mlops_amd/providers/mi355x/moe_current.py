@@ -102,27 +102,34 @@ def forward_routed(h2, residual, router_weight, w13, w2, *, top_k, routing_mode,
     with torch.no_grad():
         x = h2.reshape(rows, width).contiguous()
         base = residual.reshape(rows, width).contiguous()
-        logits = router.router_logits(x, router_weight)
         forced = next_override(rows, experts, top_k, x.device)
         bias = None if router_bias is None or router_bias.numel() == 0 else router_bias
-        weights, ids, counts, offsets, order, slots, aux, probability_sum = kernels.route(
-            logits, int(top_k), routing_mode, lengths, bias=bias, n_group=int(n_group),
-            topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced,
-        )
-        h13 = _routed_rows_gemm(x, slots, order, int(top_k), w13[0], w13[2], offsets)
+        options = dict(bias=bias, n_group=int(n_group), topk_group=int(topk_group),
+                       routed_scaling=float(routed_scaling), forced_ids=forced)
+        gathered = fused._reads_token_rows(int(top_k), w13[0].shape[1])
+        fused_routing = kernels.route_tokens(
+            x, router_weight, int(top_k), routing_mode, lengths,
+            quantize="rows" if gathered else None, **options)
+        if fused_routing is not None:
+            logits, quantized, routing = fused_routing
+        else:
+            logits, quantized = router.router_logits(x, router_weight), None
+            routing = kernels.route(logits, int(top_k), routing_mode, lengths, **options)
+        weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
+        h13 = _routed_rows_gemm(x, slots, order, int(top_k), w13[0], w13[2], offsets, quantized)
         output = kernels.moe_down(h13, w2[0], w2[2], offsets, slots, weights, base, swiglu_limit,
                                   row_scaled=True)
     return (output.reshape(h2.shape), aux, counts, probability_sum, logits, weights, ids, order,
             offsets, slots, h13)
 
 
-def _routed_rows_gemm(x, slots, order, top_k, data, scale, offsets):
+def _routed_rows_gemm(x, slots, order, top_k, data, scale, offsets, quantized=None):
     """The row-scaled GEMM on the routed rows of token rows ``x``: from
     ``GATHER_MIN_TOP_K`` routed rows per token, on the token rows quantized
     once (``mi355x_gemm_fp8_rowwise_gathered``), else on the permuted copy.
     Bitwise the same either way."""
-    if top_k >= fused.GATHER_MIN_TOP_K and data.shape[1] % 256 == 0:
-        tq, ts = kernels.quantize_rows_current(x)
+    if fused._reads_token_rows(top_k, data.shape[1]):
+        tq, ts = kernels.quantize_rows_current(x) if quantized is None else quantized
         # Routed row r reads token order[r] // top_k, divided in the kernel.
         return kernels.gemm_rowwise_gathered(tq, ts, order, data, scale, offsets,
                                              rows_div=top_k)

@@ -413,6 +413,46 @@ def test_grouped_gemm_matches_fp64(device, case):
     assert worst_cell_rel(out, want, offsets.tolist()) < 1e-2
 
 
+
+@pytest.mark.parametrize("tokens,width,experts,top_k,mode,dtype,quantize", [
+    (1, 128, 1, 1, "topk_then_softmax", torch.float32, None),        # the smallest call
+    (17, 2048, 128, 8, "topk_then_softmax", torch.float32, "blocks"),
+    (64, 4224, 40, 5, "sigmoid_noaux_tc", torch.bfloat16, "rows"),   # a last K part of 128
+    (33, 640, 9, 4, "softmax_then_topk", torch.bfloat16, "blocks"),
+    (64, 7168, 128, 16, "softmax_then_topk", torch.float32, "rows"),
+])
+def test_route_tokens_against_separate_calls(device, tokens, width, experts, top_k, mode, dtype,
+                                             quantize):
+    """The logits against the fp64 product of the bf16 operands (fp32 sums of
+    `width` products in chains of 32: 2^-24 * (32 + width / 32) of the sum of
+    magnitudes bounds them), the routing of those logits and the quantized rows
+    bitwise against the kernels called one at a time."""
+    g = torch.Generator(device=device).manual_seed(tokens + width)
+    x = torch.randn(tokens, width, generator=g, device=device).to(torch.bfloat16)
+    w = (torch.randn(experts, width, generator=g, device=device) / width ** 0.5).to(dtype)
+    bias = None
+    if mode == "sigmoid_noaux_tc":
+        bias = torch.randn(experts, generator=g, device=device) * 0.1
+    options = dict(bias=bias, routed_scaling=2.5 if bias is not None else 1.0)
+    logits, rows, routing = K.route_tokens(x, w, top_k, mode, (tokens,), quantize=quantize,
+                                           **options)
+    xd, wd = x.double(), w.to(torch.bfloat16).double()
+    bound = xd.abs() @ wd.abs().t() * 2.0 ** -24 * (32 + width / 32)
+    assert ((logits.double() - xd @ wd.t()).abs() <= bound).all()
+    for a, b in zip(routing, K.route(logits, top_k, mode, (tokens,), **options), strict=True):
+        assert torch.equal(a, b)
+    if quantize is not None:
+        q, s = (K.quantize_token_rows if quantize == "blocks" else K.quantize_rows_current)(x)
+        assert torch.equal(_bytes(rows[0]), _bytes(q)) and torch.equal(rows[1], s)
+    # Outside the range: more tokens, a group limit, sequences, an unaligned or
+    # strided operand.
+    assert K.route_tokens(x.expand(65, -1, -1)[:, 0].contiguous(), w, top_k, mode, (65,)) is None
+    assert K.route_tokens(x.repeat(2, 1), w, top_k, mode, (tokens, tokens)) is None
+    assert K.route_tokens(x, w.double(), top_k, mode, (tokens,)) is None
+    if experts > 1:
+        assert K.route_tokens(x, w.t().contiguous().t(), top_k, mode, (tokens,)) is None
+
+
 # Row counts and N that reach each tile size of the grouped GEMM: 64-row tiles
 # (few rows a group; 1 to 3 K steps, shorter than the copy pipeline), 128-row
 # tiles (129..160 rows a group), the 256 x 256 tiles, and 256 x 128 tiles (N an
