@@ -745,19 +745,33 @@ int launch(const V2Args& g, void* stream) {
 
 // Scratch for the split last round, 0 where a launch on `rows` rows is not
 // expected to have one: smaller tiles, a short K, or by the row blocks that
-// `rows` rows make on average no short last round (a second launch that finds
-// nothing to finish costs 4-6 us: hidden 4096, 14336, 8 experts at 2048 rows
-// down 201 / 207). Past ten rounds the last one is too small a share.
+// `rows` rows make no short last round (a second launch that finds nothing to
+// finish costs 4-6 us: hidden 4096, 14336, 8 experts at 2048 rows down 201 /
+// 207). The blocks are rows / 256 and half a block per expert, give or take
+// 0.29 sqrt(experts) (each expert's last block is filled evenly between 0 and
+// 1), so the rounds around the expected one count too (hidden 7168, 2048, 32
+// experts at 16384 rows, 160 tiles an XCD expected: up 687 / 672, the whole
+// forward 1-2% on three routings). Past ten rounds the last one is too small a
+// share.
 extern "C" size_t mi355x_gemm_tail_workspace_size(int rows, int experts, int n, int k) {
   if (rows <= 0 || experts <= 0 || experts > kMaxExperts || n <= 0 || n % BN != 0 || k <= 0 ||
       k % BK != 0)
     return 0;
-  const int cus = cu_count();
+  const int cus = cu_count(), n_tiles = n / BN;
   if (cus % 8 != 0 || mi355x_gemm_tile_serves(rows, experts, n)) return 0;
   const int groups = rows < experts ? rows : experts;
-  const long long tiles = ((long long)rows / BM + groups / 2) * (n / BN);
-  if (tiles > 10ll * cus || tail_split((int)(tiles / 8), cus / 8, k / BK).parts == 1) return 0;
-  return (size_t)cus * BM * BN * sizeof(float);
+  const long long tiles = ((long long)rows / BM + groups / 2) * n_tiles;
+  if (tiles > 10ll * cus) return 0;
+  int spread = 0;  // tiles an XCD: the largest s with s <= 0.29 sqrt(groups) n_tiles / 8
+  while (761ll * (spread + 1) * (spread + 1) <= (long long)groups * n_tiles * n_tiles &&
+         spread < cus / 8)
+    ++spread;
+  for (int s = -spread; s <= spread; ++s) {
+    const int mine = (int)(tiles / 8) + s;
+    if (mine > 0 && tail_split(mine, cus / 8, k / BK).parts > 1)
+      return (size_t)cus * BM * BN * sizeof(float);
+  }
+  return 0;
 }
 
 // Launches the pipelined kernel; returns 1 if the shape is not its form

@@ -601,6 +601,19 @@ def test_grouped_gemm_last_round_split_over_k(device, monkeypatch, counts, n, k)
     assert worst_cell_rel(split["rows"], product(lambda lo, hi: cd[lo:hi], rd), bounds) < 4e-3
 
 
+@pytest.mark.parametrize("rows,experts,n,k,wanted", [
+    (4096, 8, 4096, 14336, True),    # 40 tiles an XCD expected: 8 in the last round
+    (16384, 32, 4096, 7168, True),   # 160 expected, a full round; a block more leaves 2
+    (2048, 8, 4096, 14336, False),   # 24 expected, 22 to 26 likely: no half-empty round
+    (16384, 32, 7168, 2048, False),  # K too short to split
+    (640, 8, 4096, 14336, False),    # smaller tiles
+    (0, 8, 4096, 14336, False),
+])
+def test_gemm_tail_workspace_where_a_short_last_round_is_likely(device, rows, experts, n, k,
+                                                                wanted):
+    size = K._native.query("mi355x_gemm_tail_workspace_size", rows, experts, n, k)
+    assert (size > 0) == wanted
+
 
 @pytest.mark.parametrize("tokens,top_k,experts,k,n,form", [
     (2000, 4, 16, 512, 512, "up"),           # gate/up interleave, partial row tiles
