@@ -35,7 +35,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import kernels, router
+from .. import kernels
 from ..dispatch.context import weight_gradient_dtype
 from ..providers.mi355x import moe as provider
 from ..providers.mi355x import moe_current
@@ -136,15 +136,12 @@ class _ExpertLoRA(torch.autograd.Function):
         with torch.no_grad():
             x = hidden.reshape(tokens, width).contiguous()
             base = residual.reshape(tokens, width).contiguous()
-            logits = router.router_logits(x, router_weight)
             forced = next_override(tokens, experts, top_k, x.device)
-            bias = opts["router_bias"]
-            weights, ids = kernels.router_topk(
-                logits, top_k, mode, bias=bias, n_group=opts["n_group"],
-                topk_group=opts["topk_group"], routed_scaling=opts["routed_scaling"],
-                forced_ids=forced,
-            )
-            counts, offsets, order, slots = kernels.permute_plan(ids, experts)
+            logits, _, routing = provider.route_rows(
+                x, router_weight, top_k, mode, opts["lengths"], bias=opts["router_bias"],
+                n_group=opts["n_group"], topk_group=opts["topk_group"],
+                routed_scaling=opts["routed_scaling"], forced_ids=forced)
+            weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
             order_l = order.long()
             rows_token = order_l // top_k
             rows_expert = ids.reshape(-1).long()[order_l]
@@ -182,8 +179,6 @@ class _ExpertLoRA(torch.autograd.Function):
                 y = kernels.gemm(aq, as_, w2_data, w2_scale, offsets,
                                  lora=(z2p, _padded(b2b, r2)))
             output = kernels.combine(y, slots, weights, base)
-            aux, probability_sum, _, _ = kernels.router_stats(logits, ids, top_k, mode,
-                                                              opts["lengths"])
         ctx.opts = opts
         ctx.w13, ctx.w2 = w13, w2
         ctx.factor_dtypes = (a13.dtype, b13.dtype, a2.dtype, b2.dtype)

@@ -147,6 +147,19 @@ def _normalized(lengths, rows):
     return result
 
 
+def route_rows(x, router_weight, top_k, mode, lengths, *, quantize=None, **options):
+    """``(logits, rows, kernels.route's results)`` of token rows: few tokens in
+    :func:`kernels.route_tokens`, with ``rows`` their quantization, others
+    through the library GEMM (``rows`` None). Every operator routes this way,
+    so that they agree bitwise."""
+    result = kernels.route_tokens(x, router_weight, top_k, mode, lengths, quantize=quantize,
+                                  **options)
+    if result is not None:
+        return result
+    logits = router.router_logits(x, router_weight)
+    return logits, None, kernels.route(logits, top_k, mode, lengths, **options)
+
+
 def forward_routed(
     h2, residual, router_weight, w13, w2, *, top_k, routing_mode, router_bias=None,
     n_group=1, topk_group=1, routed_scaling=1.0, lengths=None, swiglu_limit=None,
@@ -167,14 +180,9 @@ def forward_routed(
         options = dict(bias=bias, n_group=int(n_group), topk_group=int(topk_group),
                        routed_scaling=float(routed_scaling), forced_ids=forced)
         gathered = _reads_token_rows(int(top_k), w13_data.shape[1])
-        fused_routing = kernels.route_tokens(
+        logits, quantized, routing = route_rows(
             x, router_weight, int(top_k), routing_mode, lengths,
             quantize="blocks" if gathered else None, **options)
-        if fused_routing is not None:
-            logits, quantized, routing = fused_routing
-        else:
-            logits, quantized = router.router_logits(x, router_weight), None
-            routing = kernels.route(logits, int(top_k), routing_mode, lengths, **options)
         weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
         # GEMM, then the SwiGLU pass: measured faster than the fused epilogue
         # of mi355x_gemm_fp8_block_swiglu, whose activation math runs while

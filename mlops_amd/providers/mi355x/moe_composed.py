@@ -30,7 +30,7 @@ from __future__ import annotations
 
 import torch
 
-from ... import kernels, router
+from ... import kernels
 from ...block_fp8 import BlockFP8Weight
 from ...dispatch import logical_costs as logical
 from ...dispatch.context import weight_gradient_dtype
@@ -125,14 +125,12 @@ def prepare_forward(h2, router_weight, w13, *, top_k, routing_mode, router_bias=
     experts = router_weight.shape[0]
     with torch.no_grad():
         x = h2.reshape(rows, width).contiguous()
-        logits = router.router_logits(x, router_weight)
         forced = next_override(rows, experts, top_k, x.device)
         bias = None if router_bias is None or router_bias.numel() == 0 else router_bias
-        weights, ids = kernels.router_topk(
-            logits, int(top_k), routing_mode, bias=bias, n_group=int(n_group),
-            topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced,
-        )
-        counts, offsets, order, slots = kernels.permute_plan(ids, experts)
+        logits, _, routing = fused.route_rows(
+            x, router_weight, int(top_k), routing_mode, lengths, bias=bias, n_group=int(n_group),
+            topk_group=int(topk_group), routed_scaling=float(routed_scaling), forced_ids=forced)
+        weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
         # Block-FP8 w13 is stored gate rows then up rows and the GEMM
         # interleaves its output; an fp8_current w13 is stored interleaved.
         if getattr(w13, "current", False):
@@ -141,8 +139,6 @@ def prepare_forward(h2, router_weight, w13, *, top_k, routing_mode, router_bias=
         else:
             h13 = fused.routed_rows_gemm(x, slots, order, int(top_k), w13, offsets,
                                          interleave=True)
-        aux, probability_sum, _, _ = kernels.router_stats(logits, ids, int(top_k), routing_mode,
-                                                          lengths)
     return aux, counts, probability_sum, logits, weights, ids, order, offsets, slots, h13
 
 

@@ -33,7 +33,7 @@ from __future__ import annotations
 
 import torch
 
-from ... import kernels, router
+from ... import kernels
 from ...block_fp8 import BlockFP8Weight
 from ...dispatch import logical_costs as logical
 from ...dispatch.context import weight_gradient_dtype
@@ -107,14 +107,9 @@ def forward_routed(h2, residual, router_weight, w13, w2, *, top_k, routing_mode,
         options = dict(bias=bias, n_group=int(n_group), topk_group=int(topk_group),
                        routed_scaling=float(routed_scaling), forced_ids=forced)
         gathered = fused._reads_token_rows(int(top_k), w13[0].shape[1])
-        fused_routing = kernels.route_tokens(
+        logits, quantized, routing = fused.route_rows(
             x, router_weight, int(top_k), routing_mode, lengths,
             quantize="rows" if gathered else None, **options)
-        if fused_routing is not None:
-            logits, quantized, routing = fused_routing
-        else:
-            logits, quantized = router.router_logits(x, router_weight), None
-            routing = kernels.route(logits, int(top_k), routing_mode, lengths, **options)
         weights, ids, counts, offsets, order, slots, aux, probability_sum = routing
         h13 = _routed_rows_gemm(x, slots, order, int(top_k), w13[0], w13[2], offsets, quantized)
         output = kernels.moe_down(h13, w2[0], w2[2], offsets, slots, weights, base, swiglu_limit,

@@ -80,6 +80,13 @@ def test_composed_equals_fused_bitwise(device, mode, kw):
     _assert_equal(fused, composed)
 
 
+@pytest.mark.parametrize("top_k", [2, 4])
+def test_composed_equals_fused_on_few_tokens(device, top_k):
+    args = _inputs(device, tokens=24, seed=5)  # the routing kernels of few tokens
+    kw = dict(top_k=top_k, routing_mode="topk_then_softmax")
+    _assert_equal(_run(FUSED, *args, **kw), _run(COMPOSED, *args, **kw))
+
+
 def test_composed_equals_fused_with_per_call_weights(device):
     """Plain bf16 masters, quantized per call (the C3 bench's weights)."""
     args = _inputs(device, tokens=384, hidden=256, experts=16, inter=128, seed=4)
