@@ -13,8 +13,9 @@
 //
 // 8 waves in a kWM x kWN grid; a wave owns MB x NB blocks of
 // v_mfma_f32_16x16x128_f8f6f4. Copies, LDS swizzle and scale folding are
-// gemm_pipe.h's. K steps run in order from 0 in every form, so all forms
-// here sum in the same order.
+// gemm_pipe.h's. A tile walks K from the step at which the 256 x 256 tile it
+// lies in would start (k_rotation), so that a row's result is the same sum in
+// the same order whichever tiles a launch uses.
 #include "gemm_pipe.h"
 
 using namespace pipe;
@@ -41,6 +42,7 @@ struct TileArgs {
   const int32_t* a_rows;
   uint32_t div_m;
   int div_s;
+  int rotate;  // start K as the 256 x 256 tiles do (N a multiple of 256)
 };
 
 // Position of 16-byte unit u in row r of a K-major stage tile (128 K rows of
@@ -86,6 +88,10 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
   __shared__ __align__(1024) uint8_t smem[kStages * STAGE];
   __shared__ int prefix[kMaxExperts + 1], starts[kMaxExperts + 1];
   __shared__ int gtok[kGather ? kTables : 1][kGather ? kBM : 1];
+  // 256-row blocks of the experts before each one: at most rows / 256 + experts,
+  // under 2^16 for the 161 rows an expert on average that choose_tiles takes.
+  // Shorts, so that two workgroups of 64-row tiles still fit a CU.
+  __shared__ uint16_t wide_prefix[kBM < 256 ? kMaxExperts : 1];
 
   const int tid = threadIdx.x, lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -97,21 +103,31 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
     int* wsum = (int*)smem;
     const int lo = tid < g.experts ? g.offsets[tid] : 0;
     const int hi = tid < g.experts ? g.offsets[tid + 1] : 0;
-    const int v = (hi - lo + kBM - 1) / kBM;
-    int x = v;
+    const int v = (hi - lo + kBM - 1) / kBM, wide = (hi - lo + BM - 1) / BM;
+    int x = v, xw = wide;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
+      const int y = __shfl_up(x, o, 64), yw = __shfl_up(xw, o, 64);
+      if (lane >= o) {
+        x += y;
+        xw += yw;
+      }
     }
-    if (lane == 63) wsum[wave] = x;
+    if (lane == 63) {
+      wsum[wave] = x;
+      wsum[kWaves + wave] = xw;
+    }
     __syncthreads();
-    int before = 0;
+    int before = 0, before_wide = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) before += w < wave ? wsum[w] : 0;
+    for (int w = 0; w < kWaves; ++w) {
+      before += w < wave ? wsum[w] : 0;
+      before_wide += w < wave ? wsum[kWaves + w] : 0;
+    }
     if (tid < g.experts) {
       prefix[tid] = before + x - v;
       starts[tid] = lo;
+      if constexpr (kBM < 256) wide_prefix[tid] = (uint16_t)(before_wide + xw - wide);
     }
     if (tid == g.experts - 1) {
       prefix[g.experts] = before + x;
@@ -136,7 +152,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
     return t < last ? t : -1;
   };
   struct Tile {
-    int e, row0, nvalid, nt;
+    int e, row0, nvalid, nt, rot;
   };
   auto describe = [&](int tile) -> Tile {
     Tile t;
@@ -150,6 +166,13 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
     const int hi = __builtin_amdgcn_readfirstlane(starts[t.e + 1]);
     t.row0 = lo + (local - t.nt * blocks) * kBM;
     t.nvalid = min(kBM, hi - t.row0);
+    t.rot = 0;
+    if constexpr (kBM < 256) {
+      if (g.rotate) {
+        const int block = wide_prefix[t.e] + (t.row0 - lo) / BM;
+        t.rot = __builtin_amdgcn_readfirstlane(k_rotation(block * (N / BN) + t.nt / (BN / TN), nk));
+      }
+    }
     return t;
   };
 
@@ -163,10 +186,11 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
     return jb < HB ? j : half_n + j;
   };
 
-  // Direct loads of K step kb of tile t into a stage; rows past the group's
-  // end repeat its last row.
+  // Direct loads of the step-th K step of tile t into a stage; rows past the
+  // group's end repeat its last row.
   const int lrow = lane >> 3, unit = (lane & 7) ^ (lane >> 3);
-  auto issue = [&](const Tile& t, int kb, int slot, int table) {
+  auto issue = [&](const Tile& t, int step, int slot, int table) {
+    const int kb = step + t.rot < nk ? step + t.rot : step + t.rot - nk;
     uint8_t* base = smem + slot * STAGE;
     const size_t koff = (size_t)kb * BK;
     const uint8_t* abase = g.a + koff + (kGather ? 0 : (size_t)t.row0 * K);
@@ -197,7 +221,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) grouped_tile_kernel(T
     uint8_t* sa = base + A_SIZE + B_SIZE;
     if constexpr (kRow) {
       // One descale per row and per column: with the tile's last step.
-      if (kb + 1 < nk) return;
+      if (step + 1 < nk) return;
       if (wave < kBM / 64) {
         const int r = wave * 64 + lane;
         uint32_t src;
@@ -525,7 +549,8 @@ int mi355x_gemm_tile_launch(const uint8_t* a, const float* a_scale, int rows, co
   const RowDiv div = row_div_magic(a_rows_div);
   const TileArgs g = {a, a_scale, rows, w, w_scale, w_scale_t, experts, n, k, offsets, interleave,
                       (const uint16_t*)addend, (uint16_t*)out, (const uint16_t*)lora_z,
-                      (const uint16_t*)lora_b, lora_rank, a_rows, div.m, div.s};
+                      (const uint16_t*)lora_b, lora_rank, a_rows, div.m, div.s,
+                      n % BN == 0 && tile_order(n, k).rotate};
   hipStream_t s = (hipStream_t)stream;
   switch (choose_tiles(rows, experts, n)) {
     // Two workgroups per CU, each with 48 KB of copies in flight.

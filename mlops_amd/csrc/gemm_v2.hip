@@ -76,19 +76,7 @@ __device__ __forceinline__ Tile describe(const int* prefix, const int32_t* __res
   }
   t.row0 = __builtin_amdgcn_readfirstlane(offsets[t.e] + (mt - prefix[t.e]) * BM);
   t.nvalid = __builtin_amdgcn_readfirstlane(min(BM, offsets[t.e + 1] - t.row0));
-  // Tiles that share an operand panel run at the same time on neighbouring
-  // CUs of one XCD; consecutive tiles start one K step apart, over a window
-  // of three steps, so that one of them takes a panel step's L2 miss and the
-  // others find the line in L2 a step later. The window is kept small: a
-  // rotation over all K steps (7t mod nk) took the same time but spread an
-  // expert's ~30 concurrent tiles over its whole 5 MB of panels, more than a
-  // 4 MB L2, and the up projection read its operands 3.6 times from HBM
-  // instead of 1.05 times (2% faster over C3's four launches). Short K
-  // (under 8 steps, e.g. the down projection) keeps the full rotation, which
-  // measured ~3% faster there, with panels small enough to stay in L2. The
-  // grouped order runs unrotated: there the CUs sharing a panel read it
-  // together.
-  t.rot = rotate ? __builtin_amdgcn_readfirstlane(nk >= 8 ? tile % 3 : (tile * 7) % nk) : 0;
+  t.rot = rotate ? __builtin_amdgcn_readfirstlane(k_rotation(tile, nk)) : 0;
   t.par = 0;
   t.steps = nk;
   return t;
@@ -669,23 +657,6 @@ __global__ void __launch_bounds__(kThreads, 2) grouped_gemm_v2_kernel(
     ct = describe_at(round, tile);
     if constexpr (kGather) ct.par = round & 1;
   }
-}
-
-// Tile order by the size of one expert's weight (N x K bytes). Up to a few
-// L2s' worth, tiles go row-block-major with the K rotation: an XCD's CUs
-// sweep one row block's N tiles, and the whole weight stays cached across
-// row blocks. Beyond that, each row block would stream the weight again
-// from HBM, so tiles go in groups of 8 N tiles x all the expert's row
-// blocks, unrotated, and the CUs that share a weight panel read it
-// together. Measured on MI355X: Mixtral's four GEMMs (58-117 MB per
-// expert) +6-14%, DeepSeek-shard up/dgrad-up (29 MB) +5-7%; the 3-15 MB
-// weights of the other shapes lose 1-7% in that order.
-struct Order {
-  int n_group, rotate;
-};
-Order tile_order(int n, int k) {
-  if ((size_t)n * (size_t)k >= ((size_t)24 << 20)) return {8, 0};
-  return {0, 1};
 }
 
 struct V2Args {

@@ -264,8 +264,12 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
   const int wm = wave >> 1, wn = wave & 1;
   const int lrow = lane >> 3, unit = (lane & 7) ^ (lane >> 3), c = lane & 15;
 
+  // Where both feature counts take 256 x 256 tiles, a tile starts at the K step
+  // at which the one it lies in would (wdescribe): one order of the sum
+  // whichever tiles compute it.
+  const int wide_n = Nf % BN == 0 && Mf % BM == 0 ? Nf / BN : 0;
   struct Tile {
-    int e, mt, nt, k0, nk;
+    int e, mt, nt, k0, nk, rot;
   };
   auto describe = [&](int tile) -> Tile {
     Tile t;
@@ -275,14 +279,20 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
     t.nt = rem - t.mt * n_tiles;
     t.k0 = __builtin_amdgcn_readfirstlane(prefix[t.e]);
     t.nk = __builtin_amdgcn_readfirstlane(prefix[t.e + 1]) - t.k0;
+    t.rot = 0;
+    if (wide_n > 0 && t.nk > 0) {
+      const int wide = (t.e * (Mf / BM) + t.mt / (BM / TM)) * wide_n + t.nt / (BN / TN);
+      t.rot = __builtin_amdgcn_readfirstlane((wide * 7) % t.nk);
+    }
     return t;
   };
-  // K block kb of tile t into a stage. The Q row behind tile row (jb, c) of a
+  // The step-th K block of tile t into a stage. The Q row behind tile row (jb, c) of a
   // wave column is feature 4c + jb of its 64, so a lane's four blocks are
   // four consecutive output columns. Scales in lane order: P's slot
   // wm * 32 + 2c + i holds row wm * 32 + 16i + c; Q's order is natural.
-  auto issue = [&](const Tile& t, int kb, int stage) {
+  auto issue = [&](const Tile& t, int step, int stage) {
     uint8_t* base = smem + stage * STAGE;
+    const int kb = step + t.rot < t.nk ? step + t.rot : step + t.rot - t.nk;
     const size_t block = (size_t)(t.k0 + kb);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {

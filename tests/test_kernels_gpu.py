@@ -526,6 +526,56 @@ def test_grouped_gemm_forms_at_every_tile_size(device, counts, n, k):
     assert worst_cell_rel(out.cpu(), want, offsets.tolist()) < 4e-3
 
 
+@pytest.mark.parametrize("counts,n,k,rows", [
+    ([1, 63, 64, 65, 0, 300, 17], 4096, 128, 2304),   # 64-row tiles; nk = 1
+    ([1, 63, 64, 65, 0, 300, 17], 4096, 384, 2304),   # nk < 8: the full rotation
+    ([1, 63, 64, 65, 0, 300, 17], 4096, 1024, 2304),  # nk >= 8: three starts
+    ([1, 63, 64, 65, 0, 300, 17], 6400, 4096, 2304),  # the large weight's order: no rotation
+    ([129, 600, 1, 0, 70], 4096, 640, 2304),          # 128-row tiles
+    ([500, 520, 500, 530, 0, 510, 1, 515], 512, 1152, 16384),  # wide grid too small
+])
+def test_small_tiles_sum_in_the_wide_tiles_order(device, monkeypatch, counts, n, k, rows):
+    """A launch on smaller tiles gives the bytes of the 256 x 256 tiles. The
+    rows of the operand, not those the offsets cover, decide the tiles, so the
+    same groups with ``rows`` operand rows run on the wide ones."""
+    monkeypatch.setattr(K, "_TAIL_MIN_K", 1 << 30)  # whole tiles on both sides
+    g = torch.Generator(device=device).manual_seed(n + k)
+    offsets = _ragged(counts).to(device)
+    used, experts, tokens = int(offsets[-1]), len(counts), 211
+    slots = torch.randint(0, 3 * tokens, (rows,), generator=g, device=device).to(torch.int32)
+    x = torch.randn(tokens, k, generator=g, device=device).to(torch.bfloat16)
+    w = (torch.randn(experts, n, k, generator=g, device=device) * 0.02).to(torch.bfloat16)
+    tq, ts = K.quantize_token_rows(x)
+    ctq, cts = K.quantize_rows_current(x)
+    wq, ws = K.quantize_weight_blocks(w)
+    kq, ks = K.quantize_weight_blocks(w.transpose(1, 2).contiguous())
+    rq, _, rs, _ = K.quantize_weights_current(w)
+    b = (torch.randn(experts, n, 16, generator=g, device=device) * 0.1).to(torch.bfloat16)
+    z = (torch.randn(rows, 16, generator=g, device=device) * 0.5).to(torch.bfloat16)
+
+    def forms(count):
+        routed = x[(slots[:count] // 3).long()]
+        xq, xs = K.quantize_rows(routed)
+        cq, cs = K.quantize_rows_current(routed)
+        return dict(
+            plain=K.gemm(xq, xs, wq, ws, offsets),
+            interleaved=K.gemm(xq, xs, wq, ws, offsets, interleave=True),
+            rank=K.gemm(xq, xs, wq, ws, offsets, lora=(z[:count], b)),
+            gathered=K.gemm_gathered(tq, ts, slots[:count], wq, ws, offsets, rows_div=3),
+            kmajor=K.gemm_kmajor(xq, xs, kq, ks, offsets),
+            kmajor_gathered=K.gemm_gathered(tq, ts, slots[:count], kq, ks, offsets, kmajor=True,
+                                            rows_div=3),
+            rows=K.gemm_rowwise(cq, cs, rq, rs, offsets),
+            rows_rank=K.gemm_rowwise(cq, cs, rq, rs, offsets, lora=(z[:count], b)),
+            rows_gathered=K.gemm_rowwise_gathered(ctq, cts, slots[:count], rq, rs, offsets,
+                                                  rows_div=3),
+        )
+
+    small, wide = forms(used), forms(rows)
+    for name, out in small.items():
+        assert torch.equal(out, wide[name][:used]), name
+
+
 @pytest.mark.parametrize("counts,n,k", [
     ([300, 511, 0, 900, 130], 8192, 4096),  # a full round, then 4 tiles an XCD in 4 parts
     ([500, 400, 300, 500], 4096, 8192),  # fewer tiles than CUs: 16 an XCD in 2 parts
@@ -879,6 +929,26 @@ def test_wgrad_at_both_tile_sizes(device, out_dtype, counts, features):
             assert torch.all(out[e] == 0)
             continue
         assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_wgrad_small_tiles_sum_in_the_wide_tiles_order(device, out_dtype):
+    """The 128 x 128 tiles give the bytes of the 256 x 256 ones where both
+    serve the widths. Empty experts behind the others add tiles, and with them
+    the wide kernel, without moving a row."""
+    counts, m, n, more = [1200, 0, 130, 1, 700, 384], 512, 768, 60
+    g = torch.Generator().manual_seed(23)
+    offsets = _ragged(counts)
+    rows = int(offsets[-1])
+    many = torch.cat([offsets, offsets[-1:].expand(more)]).contiguous().to(device)
+    padded = K.wgrad_padded_rows(rows, len(counts) + more)
+    operands = []
+    for width in (m, n):
+        x = torch.randn(rows, width, generator=g).to(torch.bfloat16).to(device)
+        operands += K.quantize_transpose(x, offsets.to(device), rows, padded=padded)[:2]
+    small = K.wgrad(*operands, offsets.to(device), out_dtype=out_dtype)
+    wide = K.wgrad(*operands, many, out_dtype=out_dtype)
+    assert torch.equal(small, wide[:len(counts)])
 
 
 def test_combine_and_token_sum(device):
