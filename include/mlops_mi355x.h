@@ -512,9 +512,11 @@ int mi355x_gemm_fp8(const mi355x_gemm_args* args, void* stream);
  *   out[e][m][n] = sum_{rows of e} p[m][row] q[n][row], block-scaled,
  * fp32 accumulation, written as bf16 (out_fp32 == 0) or fp32. p_scale
  * [padded/128][m_features], q_scale [padded/128][n_features]: powers of two
- * (as written by mi355x_quantize_transpose_fp8; the MFMA applies them in
- * hardware, by their exponents). Experts with no rows get zeros. Replaces the varlen-K wgrad GEMMs
- * (providers/sonicmoe/moe.py:351-365, :404-419; quack_moe/wgrad.py:30). */
+ * (as written by mi355x_quantize_transpose_fp8; other values are truncated to
+ * their power-of-two exponent when both feature counts are multiples of 256,
+ * where the MFMA applies the scales in hardware, and applied as they are at
+ * other widths). Experts with no rows get zeros. Replaces the varlen-K wgrad
+ * GEMMs (providers/sonicmoe/moe.py:351-365, :404-419; quack_moe/wgrad.py:30). */
 int mi355x_gemm_fp8_block_wgrad(const uint8_t* p, const float* p_scale, int m_features,
                                 const uint8_t* q, const float* q_scale, int n_features,
                                 int padded, const int32_t* offsets, int experts, void* out,

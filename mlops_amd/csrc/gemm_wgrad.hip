@@ -34,6 +34,25 @@ __device__ __forceinline__ int feature_col(int tr, int nt) {
 
 __device__ __forceinline__ int e8m0(float pow2_scale) { return __float_as_int(pow2_scale) >> 23; }
 
+// Whether E8M0 holds every scale added: positive normal powers of two.
+struct ScalesSeen {
+  uint32_t any = 0, least = 0x7f000000u, most = 0;  // bits OR-ed, their minimum, maximum
+  __device__ __forceinline__ void add(float s) {
+    const uint32_t bits = __float_as_uint(s);
+    any |= bits;
+    least = min(least, bits);
+    most = max(most, bits);
+  }
+  template <typename... Rest>
+  __device__ __forceinline__ void add(float s, Rest... rest) {
+    add(s);
+    add(rest...);
+  }
+  __device__ __forceinline__ bool e8m0() const {
+    return (any & 0x807fffffu) == 0 && least >= 0x00800000u && most < 0x7f800000u;
+  }
+};
+
 __device__ __forceinline__ v4f mfma_e8(v8i a, v8i b, v4f c, int sa, int sb) {
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, sa, 0, sb);
 }
@@ -239,15 +258,31 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
 // steps and its output decides (a 256 x 256 tile's epilogue then runs alone
 // on its CU; two workgroups overlap one's stores with the other's copies).
 // 8 waves in a 4 x 2 grid, wave tile 32 x 64 (2 x 4 blocks), two stages.
+//
+// kAnyScale: widths that the 256 x 256 tiles do not take apply any fp32 scale.
+// The transposing quantizer writes powers of two, so the loop lets the MFMA
+// apply them as above and only gathers what it saw of them (nine VALU
+// instructions a step); a wave that met others forms its part of the tile
+// again, straight from memory, folding each step's raw product into the sums
+// with FMAs. 1280 x 1152 and 1152 x 640, 16 experts, 12004 rows, fp32 out, us:
+// 37-39 and 21 without the look, 38 and 21 with it (bf16 30 and 17, 31 and 17),
+// 127 and 69 where every scale is another. (A branch in the K loop took 42 and
+// 23 with powers of two: its waits come before the fragment reads, or it spills.)
 namespace small {
 constexpr int TM = 128, TN = 128;
 constexpr int MB = 2, NB = 4;
 constexpr int A_SIZE = TM * BK, B_SIZE = TN * BK;
 constexpr int STAGE = A_SIZE + B_SIZE + 4 * (TM + TN);
 constexpr int kStores = MB * 4;  // store instructions of a wave's epilogue
+
+// frag() of one operand row's K block in memory: its units g and g + 4.
+__device__ __forceinline__ v8i frag_global(const uint8_t* block, int g) {
+  const uint4 x = *(const uint4*)(block + 16 * g), y = *(const uint4*)(block + 64 + 16 * g);
+  return (v8i){(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)y.x, (int)y.y, (int)y.z, (int)y.w};
+}
 }  // namespace small
 
-template <bool kFp32>
+template <bool kFp32, bool kAnyScale>
 __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
     const uint8_t* __restrict__ p, const float* __restrict__ p_scale, int Mf,
     const uint8_t* __restrict__ q, const float* __restrict__ q_scale, int Nf, int padded,
@@ -376,6 +411,7 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
     const int tile = tile_at(round);
     if (tile < 0) break;
     const Tile ct = describe(tile);
+    ScalesSeen seen;
     v4f acc[MB][NB];
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -401,12 +437,45 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
       for (int i = 0; i < MB; ++i) af[i] = frag(ta, (wm * MB + i) * 16 + c, lane);
 #pragma unroll
       for (int j = 0; j < NB; ++j) bf[j] = frag(tb, (wn * NB + j) * 16 + c, lane);
+      if constexpr (kAnyScale) seen.add(sa2.x, sa2.y, sb4.x, sb4.y, sb4.z, sb4.w);
       const int ea[MB] = {e8m0(sa2.x), e8m0(sa2.y)};
       const int eb[NB] = {e8m0(sb4.x), e8m0(sb4.y), e8m0(sb4.z), e8m0(sb4.w)};
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int i = 0; i < MB; ++i) acc[i][j] = mfma_e8(af[i], bf[j], acc[i][j], ea[i], eb[j]);
+    }
+    if (kAnyScale && !__all(seen.e8m0())) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+      const int g = lane >> 4, prow = ct.mt * TM + wm * 32, qrow = ct.nt * TN + wn * 64 + 4 * c;
+#pragma unroll 1
+      for (int kb = 0; kb < ct.nk; ++kb) {
+        const size_t block = (size_t)(ct.k0 + kb);
+        v8i af[MB];
+        float4 rs[MB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          af[i] = frag_global(p + (size_t)(prow + i * 16 + c) * padded + block * 128, g);
+          rs[i] = *(const float4*)(p_scale + block * Mf + prow + i * 16 + 4 * g);
+        }
+        const float4 cs = *(const float4*)(q_scale + block * Nf + qrow);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const v8i bf = frag_global(q + (size_t)(qrow + j) * padded + block * 128, g);
+          const float s = j == 0 ? cs.x : j == 1 ? cs.y : j == 2 ? cs.z : cs.w;
+#pragma unroll
+          for (int i = 0; i < MB; ++i) {
+            const v4f raw = mfma(af[i], bf);
+            acc[i][j][0] = fmaf(raw[0], rs[i].x * s, acc[i][j][0]);
+            acc[i][j][1] = fmaf(raw[1], rs[i].y * s, acc[i][j][1]);
+            acc[i][j][2] = fmaf(raw[2], rs[i].z * s, acc[i][j][2]);
+            acc[i][j][3] = fmaf(raw[3], rs[i].w * s, acc[i][j][3]);
+          }
+        }
+      }
     }
     const size_t row0 = (size_t)ct.e * Mf + ct.mt * TM + wm * 32;
     const size_t col0 = (size_t)ct.nt * TN + wn * 64 + c * 4;
@@ -438,7 +507,7 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
 // experts (128 and 512 tiles) 22 / 15 at 2048 tokens and 60 / 37 at 8192.
 // The 128 x 128 kernel it replaces at other widths, with register-staged
 // copies and a VALU fold of the scales, took 271 us for the two gradients of
-// 1152 x 1280 and 640, 16 experts, 12004 rows in fp32; this one takes 62.
+// 1152 x 1280 and 640, 16 experts, 12004 rows in fp32; this one takes 59.
 int mi355x_wgrad_launch(const uint8_t* p, const float* p_scale, int m_features, const uint8_t* q,
                         const float* q_scale, int n_features, int padded, const int32_t* offsets,
                         int experts, void* out, int out_fp32, void* stream) {
@@ -455,7 +524,9 @@ int mi355x_wgrad_launch(const uint8_t* p, const float* p_scale, int m_features, 
                        m_features, q, q_scale, n_features, padded, offsets, experts, out);
   };
   if (wide) out_fp32 ? launch(wgrad_v2_kernel<true>) : launch(wgrad_v2_kernel<false>);
-  else out_fp32 ? launch(wgrad_tile_kernel<true>) : launch(wgrad_tile_kernel<false>);
+  else if (m_features % BM == 0 && n_features % BN == 0)
+    out_fp32 ? launch(wgrad_tile_kernel<true, false>) : launch(wgrad_tile_kernel<false, false>);
+  else out_fp32 ? launch(wgrad_tile_kernel<true, true>) : launch(wgrad_tile_kernel<false, true>);
   MI355X_LAUNCH_CHECK();
   return MI355X_OK;
 }

@@ -931,6 +931,37 @@ def test_wgrad_at_both_tile_sizes(device, out_dtype, counts, features):
         assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
 
 
+@pytest.mark.parametrize("features", [(128, 384), (256, 640), (384, 512)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_wgrad_applies_any_scale_at_odd_widths(device, out_dtype, features):
+    """Descales that are no powers of two, and zeros, at widths outside the
+    256 x 256 tiles, against the fp64 sums; the bounds of
+    test_wgrad_at_both_tile_sizes hold (the fold of a step is one more fp32
+    rounding of its product, 2^-24). Some steps keep power-of-two scales, so
+    one tile's sum mixes both ways of applying them."""
+    counts = [300, 0, 1, 513]
+    g = torch.Generator().manual_seed(sum(features))
+    offsets = _ragged(counts)
+    rows = int(offsets[-1])
+    padded = K.wgrad_padded_rows(rows, len(counts))
+    operands = []
+    for width in features:
+        x = torch.randn(rows, width, generator=g).to(torch.bfloat16).to(device)
+        q, s, _ = K.quantize_transpose(x, offsets.to(device), rows, padded=padded)
+        factor = torch.rand(s.shape, generator=g) + 0.5
+        factor[1] = 1.0
+        factor[3, ::7] = 0.0
+        operands += [q, s * factor.to(device)]
+    out = K.wgrad(*operands, offsets.to(device), out_dtype=out_dtype).cpu()
+    want = O.wgrad(*(t.cpu() for t in operands), offsets)
+    tol = 6e-5 if out_dtype == torch.float32 else 4e-3
+    for e, n in enumerate(counts):
+        if n == 0:
+            assert torch.all(out[e] == 0)
+            continue
+        assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
+
+
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_wgrad_small_tiles_sum_in_the_wide_tiles_order(device, out_dtype):
     """The 128 x 128 tiles give the bytes of the 256 x 256 ones where both
