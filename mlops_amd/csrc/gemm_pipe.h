@@ -57,6 +57,11 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, const uint
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds_addr(lds)), "v"(off), "s"(base) : "memory", "m0");
 }
+// The same from a per-lane 64-bit address, for rows too far apart for an offset.
+__device__ __forceinline__ void dma16_far(const uint8_t* src, const uint8_t* lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(lds_addr(lds)), "v"(src) : "memory", "m0");
+}
 __device__ __forceinline__ void dma4(const void* base, uint32_t off, const uint8_t* lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :: "s"(lds_addr(lds)), "v"(off), "s"(base) : "memory", "m0");

@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(kThreads, 2) wgrad_v2_kernel(
 // on its CU; two workgroups overlap one's stores with the other's copies).
 // 8 waves in a 4 x 2 grid, wave tile 32 x 64 (2 x 4 blocks), two stages.
 //
-// kAnyScale: widths that the 256 x 256 tiles do not take apply any fp32 scale.
+// kAnyScale: shapes that the 256 x 256 tiles do not take apply any fp32 scale.
 // The transposing quantizer writes powers of two, so the loop lets the MFMA
 // apply them as above and only gathers what it saw of them (nine VALU
 // instructions a step); a wave that met others forms its part of the tile
@@ -274,6 +274,9 @@ constexpr int MB = 2, NB = 4;
 constexpr int A_SIZE = TM * BK, B_SIZE = TN * BK;
 constexpr int STAGE = A_SIZE + B_SIZE + 4 * (TM + TN);
 constexpr int kStores = MB * 4;  // store instructions of a wave's epilogue
+// kFar: from here on 28 padded rows exceed a 32-bit offset. Not a branch in the
+// kernel, which costs the ordinary launch 6%.
+constexpr int kFarRows = 1 << 27;
 
 // frag() of one operand row's K block in memory: its units g and g + 4.
 __device__ __forceinline__ v8i frag_global(const uint8_t* block, int g) {
@@ -282,7 +285,7 @@ __device__ __forceinline__ v8i frag_global(const uint8_t* block, int g) {
 }
 }  // namespace small
 
-template <bool kFp32, bool kAnyScale>
+template <bool kFp32, bool kAnyScale, bool kFar>
 __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
     const uint8_t* __restrict__ p, const float* __restrict__ p_scale, int Mf,
     const uint8_t* __restrict__ q, const float* __restrict__ q_scale, int Nf, int padded,
@@ -325,6 +328,10 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
   // wave column is feature 4c + jb of its 64, so a lane's four blocks are
   // four consecutive output columns. Scales in lane order: P's slot
   // wm * 32 + 2c + i holds row wm * 32 + 16i + c; Q's order is natural.
+  auto copy = [&](const uint8_t* base, int row, uint8_t* to) {
+    if constexpr (kFar) dma16_far(base + (size_t)row * padded + 16 * unit, to);
+    else dma16(base, (uint32_t)row * (uint32_t)padded + 16 * unit, to);
+  };
   auto issue = [&](const Tile& t, int step, int stage) {
     uint8_t* base = smem + stage * STAGE;
     const int kb = step + t.rot < t.nk ? step + t.rot : step + t.rot - t.nk;
@@ -332,15 +339,13 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int tr = (wave * 2 + i) * 8;
-      dma16(p + (size_t)(t.mt * TM + tr) * padded + block * 128,
-            (uint32_t)lrow * (uint32_t)padded + 16 * unit, base + tr * 128);
+      copy(p + (size_t)(t.mt * TM + tr) * padded + block * 128, lrow, base + tr * 128);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int tr = (wave * 2 + i) * 8;
       const int feature = t.nt * TN + (tr >> 6) * 64 + (tr & 8) * 4 + ((tr >> 4) & 3);
-      dma16(q + (size_t)feature * padded + block * 128,
-            (uint32_t)(4 * lrow) * (uint32_t)padded + 16 * unit, base + A_SIZE + tr * 128);
+      copy(q + (size_t)feature * padded + block * 128, 4 * lrow, base + A_SIZE + tr * 128);
     }
     uint8_t* scales = base + A_SIZE + B_SIZE;
     if (wave < 2) {
@@ -500,8 +505,9 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
 
 }  // namespace
 
-// 256 x 256 tiles where both feature counts are multiples of 256 and the tiles
-// fill the CUs at least once, else 128 x 128 tiles. Measured on MI355X (256-
+// 256 x 256 tiles where both feature counts are multiples of 256, 32-bit
+// offsets reach the operands and the tiles fill the CUs at least once, else
+// 128 x 128 tiles. Measured on MI355X (256-
 // / 128-sided tiles, bf16 out, us): 2048 x 1536, 128 experts 135 / 144 at 1021
 // tokens (0.8 GB written, 5.9 TB/s) and 486 / 654 at 16384; 2048 x 512, 8
 // experts (128 and 512 tiles) 22 / 15 at 2048 tokens and 60 / 37 at 8192.
@@ -511,11 +517,11 @@ __global__ void __launch_bounds__(kThreads, 4) wgrad_tile_kernel(
 int mi355x_wgrad_launch(const uint8_t* p, const float* p_scale, int m_features, const uint8_t* q,
                         const float* q_scale, int n_features, int padded, const int32_t* offsets,
                         int experts, void* out, int out_fp32, void* stream) {
-  bool wide = m_features % BM == 0 && n_features % BN == 0 &&
-              (uint64_t)m_features * (uint64_t)padded < (1ull << 32) &&
-              (uint64_t)n_features * (uint64_t)padded < (1ull << 32);
-  wide = wide && (long long)experts * (m_features / BM) * (n_features / BN) >= cu_count();
-  MI355X_REQUIRE(wide || (uint64_t)padded < (1ull << 27), "wgrad: padded rows beyond 2^27");
+  const bool fits = m_features % BM == 0 && n_features % BN == 0 &&
+                    (uint64_t)m_features * (uint64_t)padded < (1ull << 32) &&
+                    (uint64_t)n_features * (uint64_t)padded < (1ull << 32);
+  const bool wide =
+      fits && (long long)experts * (m_features / BM) * (n_features / BN) >= cu_count();
   const int side = wide ? BM : small::TM, slots = wide ? cu_count() : 2 * cu_count();
   const long long total = (long long)experts * (m_features / side) * (n_features / side);
   const int grid = total < slots ? (int)total : slots;
@@ -524,9 +530,15 @@ int mi355x_wgrad_launch(const uint8_t* p, const float* p_scale, int m_features, 
                        m_features, q, q_scale, n_features, padded, offsets, experts, out);
   };
   if (wide) out_fp32 ? launch(wgrad_v2_kernel<true>) : launch(wgrad_v2_kernel<false>);
-  else if (m_features % BM == 0 && n_features % BN == 0)
-    out_fp32 ? launch(wgrad_tile_kernel<true, false>) : launch(wgrad_tile_kernel<false, false>);
-  else out_fp32 ? launch(wgrad_tile_kernel<true, true>) : launch(wgrad_tile_kernel<false, true>);
+  else if (fits)
+    out_fp32 ? launch(wgrad_tile_kernel<true, false, false>)
+             : launch(wgrad_tile_kernel<false, false, false>);
+  else if (padded < small::kFarRows)
+    out_fp32 ? launch(wgrad_tile_kernel<true, true, false>)
+             : launch(wgrad_tile_kernel<false, true, false>);
+  else
+    out_fp32 ? launch(wgrad_tile_kernel<true, true, true>)
+             : launch(wgrad_tile_kernel<false, true, true>);
   MI355X_LAUNCH_CHECK();
   return MI355X_OK;
 }

@@ -962,6 +962,27 @@ def test_wgrad_applies_any_scale_at_odd_widths(device, out_dtype, features):
         assert worst_cell_rel(out[e], want[e], list(range(0, features[0] + 1, 128))) < tol, e
 
 
+def test_wgrad_rows_beyond_32_bit_offsets(device):
+    """A padded row count whose feature rows lie further apart than a 32-bit
+    offset spans (two operands of 20 GB, their first two row blocks filled)
+    gives the bytes of the same rows in a short layout."""
+    features, padded, rows = (128, 128), 160_000_000, 200
+    offsets = torch.tensor([0, rows], dtype=torch.int32, device=device)
+    g = torch.Generator().manual_seed(29)
+    short, far = [], []
+    for width in features:
+        x = torch.randn(rows, width, generator=g).to(torch.bfloat16).to(device)
+        q, s, _ = K.quantize_transpose(x, offsets, rows, padded=256)
+        wide_q = torch.empty(width, padded, dtype=K.FP8, device=device)
+        wide_s = torch.empty(padded // 128, width, dtype=torch.float32, device=device)
+        wide_q.view(torch.uint8)[:, :256] = q.view(torch.uint8)
+        wide_s[:2] = s
+        short += [q, s]
+        far += [wide_q, wide_s]
+    want = K.wgrad(*short, offsets, out_dtype=torch.float32)
+    assert torch.equal(K.wgrad(*far, offsets, out_dtype=torch.float32), want)
+
+
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_wgrad_small_tiles_sum_in_the_wide_tiles_order(device, out_dtype):
     """The 128 x 128 tiles give the bytes of the 256 x 256 ones where both
