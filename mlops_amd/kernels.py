@@ -1102,6 +1102,8 @@ def route_tokens(x, weight, top_k: int, mode: str, lengths: Sequence[int], *, bi
     tokens, width = x.shape
     if tokens > _ROUTE_TOKENS or len(lengths) > 1 or mode not in ROUTING_MODES:
         return None
+    if weight.ndim != 2 or weight.shape[1] != width:
+        return None  # the library GEMM refuses it
     if (x.dtype != torch.bfloat16 or weight.dtype not in (torch.float32, torch.bfloat16)
             or weight.device != x.device or not x.is_contiguous() or not weight.is_contiguous()
             or (x.data_ptr() | weight.data_ptr()) & 15):

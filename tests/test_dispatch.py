@@ -473,3 +473,17 @@ def test_implementation_pairs():
     # The MoE catalog has no plain-torch record: the hot path has no fallback.
     with pytest.raises(ValueError, match="no native_torch"):
         implementation_pairs(["moe"])
+
+
+def test_few_token_routing_leaves_a_mismatched_router_weight_to_the_gemm():
+    """The routing kernel reads the weight as ``[E, width]`` by pointer: a weight
+    of another shape, which a call below the registry's support check can bring,
+    goes to the library GEMM and its error."""
+    from mlops_amd import kernels
+
+    x = torch.zeros(4, 256, dtype=torch.bfloat16)
+    for shape in ((8, 128), (8, 512), (8,), (8, 256, 1)):
+        weight = torch.zeros(shape)
+        assert kernels.route_tokens(x, weight, 2, "topk_then_softmax", (4,)) is None
+        with pytest.raises(RuntimeError):
+            provider.route_rows(x, weight, 2, "topk_then_softmax", (4,))
