@@ -504,6 +504,7 @@ typedef struct mi355x_gemm_args {
   int32_t rows, a_total, a_rows_div, experts, n, k;
   int32_t w_scale_t, interleave, row_scaled, kmajor, lora_rank;
 } mi355x_gemm_args;
+size_t mi355x_gemm_args_size(void); /* sizeof(mi355x_gemm_args), for other languages' bindings */
 size_t mi355x_gemm_tail_workspace_size(int rows, int experts, int n, int k);
 int mi355x_gemm_fp8(const mi355x_gemm_args* args, void* stream);
 
@@ -597,6 +598,7 @@ typedef struct mi355x_moe_block_bwd_args {
   int32_t tokens, hidden, inter, experts, top_k, mode, segments, w13_kmajor, weight_grads_fp32;
   float limit;
 } mi355x_moe_block_bwd_args;
+size_t mi355x_moe_block_bwd_args_size(void); /* sizeof(mi355x_moe_block_bwd_args) */
 size_t mi355x_moe_block_bwd_workspace_size(int tokens, int hidden, int inter, int experts,
                                            int top_k, int need_w13, int need_w2,
                                            int router_kernel);

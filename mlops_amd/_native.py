@@ -7,6 +7,7 @@ missing or a GPU entry point fails, the error says so and nothing else runs.
 from __future__ import annotations
 
 import ctypes
+import struct
 import threading
 from pathlib import Path
 
@@ -108,10 +109,17 @@ SIGNATURES = {
     "mi355x_moe_down": (_I, [_P, _I, _I, _I, _I, _F, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _S,
                              _P]),
     "mi355x_moe_block_bwd_workspace_size": (_S, [_I] * 8),
+    "mi355x_moe_block_bwd_args_size": (_S, []),
     "mi355x_moe_block_bwd": (_I, [ctypes.c_char_p, _P]),  # the packed argument struct
     "mi355x_gemm_tail_workspace_size": (_S, [_I] * 4),
+    "mi355x_gemm_args_size": (_S, []),
     "mi355x_gemm_fp8": (_I, [ctypes.c_char_p, _P]),  # the packed argument struct
 }
+
+# The argument structs as the entry points read them, tail padding included;
+# library() holds their sizes against the C ones.
+GEMM_ARGS = struct.Struct("=12Q11i4x")  # 11 pointers, the workspace size, eleven ints
+MOE_BLOCK_BWD_ARGS = struct.Struct("=23Q9if")  # 22 pointers, the size, nine ints, a float
 
 _lock = threading.Lock()
 _lib = None
@@ -138,6 +146,11 @@ def library() -> ctypes.CDLL:
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes
+            for packed, size in ((GEMM_ARGS, lib.mi355x_gemm_args_size()),
+                                 (MOE_BLOCK_BWD_ARGS, lib.mi355x_moe_block_bwd_args_size())):
+                if packed.size != size:
+                    raise RuntimeError(f"{LIBRARY.name}: an argument struct of {size} bytes is "
+                                       f"packed as {packed.size}; rebuild the library")
             _lib = lib
     return _lib
 
@@ -156,4 +169,5 @@ def query(name: str, *args) -> int:
     return int(getattr(library(), name)(*args))
 
 
-__all__ = ["LIBRARY", "NativeError", "SIGNATURES", "call", "library", "query"]
+__all__ = ["GEMM_ARGS", "LIBRARY", "MOE_BLOCK_BWD_ARGS", "NativeError", "SIGNATURES", "call",
+           "library", "query"]

@@ -176,6 +176,8 @@ int rowwise(const mi355x_gemm_args& g, void* stream) {
 
 }  // namespace
 
+extern "C" size_t mi355x_gemm_args_size(void) { return sizeof(mi355x_gemm_args); }
+
 extern "C" int mi355x_gemm_fp8(const mi355x_gemm_args* args, void* stream) {
   MI355X_REQUIRE(args != nullptr, "gemm: no arguments");
   mi355x_gemm_args g = *args;

@@ -237,6 +237,10 @@ extern "C" size_t mi355x_moe_block_bwd_workspace_size(int tokens, int hidden, in
                         router_kernel).total;
 }
 
+extern "C" size_t mi355x_moe_block_bwd_args_size(void) {
+  return sizeof(mi355x_moe_block_bwd_args);
+}
+
 extern "C" int mi355x_moe_block_bwd(const mi355x_moe_block_bwd_args* a, void* stream) {
   MI355X_REQUIRE(a != nullptr && a->tokens >= 0 && a->top_k > 0 && a->hidden > 0 && a->inter > 0 &&
                      a->inter % 128 == 0 && a->hidden % 128 == 0 && a->experts > 0,

@@ -12,7 +12,6 @@ Layouts: routed rows ``A = tokens * top_k`` are in expert-sorted order;
 from __future__ import annotations
 
 import ctypes
-import struct
 from typing import Sequence
 
 import torch
@@ -593,8 +592,6 @@ def swiglu_bwd_bf16(r, h, weights, order, offsets, *, padded, row_blocks, limit=
 
 
 # ------------------------------------------------------------------- GEMMs
-# mi355x_gemm_args: 11 pointers, the workspace size, eleven ints.
-_GEMM_ARGS = struct.Struct("=12Q11i")
 _TAIL_MIN_K = 4096  # a shorter K is never split (mi355x_gemm_tail_workspace_size is 0)
 
 
@@ -618,7 +615,7 @@ def _run_gemm(name, entry, arguments, a, a_scale, w, w_scale, offsets, out, k, *
         _timed(name, device, flops, nbytes, entry, *arguments, _stream(device))
         return out
     workspace = torch.empty(size, dtype=torch.uint8, device=device)
-    packed = _GEMM_ARGS.pack(
+    packed = _native.GEMM_ARGS.pack(
         *(0 if t is None else t.data_ptr()
           for t in (a, a_scale, a_rows, w, w_scale, offsets, addend, z, b, out, workspace)),
         size, rows, a_total, a_rows_div, experts, n, k, int(transposed_scale), int(interleave),
@@ -1183,10 +1180,6 @@ def moe_down(h13, w2, w2_scale, offsets, slots, weights, residual, limit=None, *
     return out
 
 
-# mi355x_moe_block_bwd_args: 22 pointers, the workspace size, nine ints, a float.
-_BACKWARD_ARGS = struct.Struct("=23Q9if")
-
-
 def router_grad_on_kernel(x, experts: int) -> bool:
     """Whether ``mi355x_router_weight_grad`` forms the router weight gradient:
     fewer than 64 experts would leave most of its 128-expert tile idle."""
@@ -1271,7 +1264,7 @@ def moe_block_backward(r, h13, x, dy, logits, route_weights, route_ids, order, o
         r, h13, x, dy, logits, route_weights, route_ids, order, offsets, slots, w13, w13_scale,
         grad_aux, grad_prob_sum, seg_offsets, seg_counts, grad_x, pieces, grad_w13, grad_w2,
         grad_router, work)]
-    _native.call("mi355x_moe_block_bwd", _BACKWARD_ARGS.pack(
+    _native.call("mi355x_moe_block_bwd", _native.MOE_BLOCK_BWD_ARGS.pack(
         *pointers, size, tokens, hidden, inter, experts, top_k, ROUTING_MODES[mode],
         1 if seg_counts is None else seg_counts.shape[0], int(w13_kmajor), int(fp32),
         _limit(limit)), _stream(device))

@@ -56,6 +56,12 @@ def test_validation_errors(name, args, message):
         _native.call(name, *args)
 
 
+def test_packed_argument_structs_cover_the_c_ones():
+    """The entry points copy the whole struct, tail padding included."""
+    assert _native.GEMM_ARGS.size == _native.query("mi355x_gemm_args_size")
+    assert _native.MOE_BLOCK_BWD_ARGS.size == _native.query("mi355x_moe_block_bwd_args_size")
+
+
 def test_sizes_are_queries():
     assert _native.query("mi355x_wgrad_padded_rows", 1000, 8) % 128 == 0
     assert _native.query("mi355x_wgrad_padded_rows", 1000, 8) >= 1000 + 8 * 127
