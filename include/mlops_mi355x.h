@@ -499,7 +499,7 @@ typedef struct mi355x_gemm_args {
   const void* lora_z;      /* with lora_rank, else NULL */
   const void* lora_b;
   void* out;               /* bf16 [rows, N] */
-  void* workspace;         /* or NULL */
+  void* workspace;         /* 16-byte aligned, or NULL */
   uint64_t workspace_bytes;
   int32_t rows, a_total, a_rows_div, experts, n, k;
   int32_t w_scale_t, interleave, row_scaled, kmajor, lora_rank;
@@ -527,6 +527,7 @@ int mi355x_gemm_fp8_block_wgrad(const uint8_t* p, const float* p_scale, int m_fe
 
 /* Launch sequences of one layer pass: the entry points above, in order, from
  * one call and one workspace (each the same kernels, arguments and results).
+ * A workspace holds their buffers and must be 16-byte aligned.
  *
  * mi355x_moe_route: router_topk, permute_plan and router_stats on the logits
  * (moe_router.py:235-344; moe_dispatch.py:106-119; moe_common.py:32-71).

@@ -193,6 +193,8 @@ extern "C" int mi355x_gemm_fp8(const mi355x_gemm_args* args, void* stream) {
   if (g.workspace != nullptr) {
     const size_t size = mi355x_gemm_tail_workspace_size(g.rows, g.experts, g.n, g.k);
     MI355X_REQUIRE(g.workspace_bytes >= size, "gemm: workspace too small");
+    MI355X_REQUIRE(size == 0 || ((uintptr_t)g.workspace & 15) == 0,
+                   "gemm: the workspace must be 16-byte aligned");
     if (size == 0) g.workspace = nullptr;
   }
   if (g.kmajor) return kmajor(g, stream);

@@ -138,6 +138,8 @@ extern "C" int mi355x_moe_route(const float* logits, int tokens, int experts, in
   MI355X_REQUIRE(tokens >= 0 && experts > 0 && top_k > 0, "moe_route: bad sizes");
   const RouteSpace s = route_space(workspace, tokens, experts, top_k, segments, nchunks);
   MI355X_REQUIRE(workspace_bytes >= s.total, "moe_route: workspace too small");
+  MI355X_REQUIRE(((uintptr_t)workspace & 15) == 0,
+                 "moe_route: the workspace must be 16-byte aligned");
   const int small = mi355x_route_small((float*)logits, nullptr, 0, tokens, experts, top_k, mode,
                                        bias, n_group, topk_group, routed_scaling, forced_ids,
                                        segments, weights, ids, counts, offsets, order, slots, aux,
@@ -205,6 +207,8 @@ extern "C" int mi355x_moe_down(const void* h13, int tokens, int top_k, int hidde
   const int rows = tokens * top_k;
   const DownSpace s = down_space(workspace, rows, hidden, inter, experts);
   MI355X_REQUIRE(workspace_bytes >= s.total, "moe_down: workspace too small");
+  MI355X_REQUIRE(((uintptr_t)workspace & 15) == 0,
+                 "moe_down: the workspace must be 16-byte aligned");
   if (row_scaled)
     STEP(mi355x_swiglu_quantize_rows_current_fp8(h13, rows, inter, limit, s.q, s.scales, nullptr,
                                                  stream));
@@ -251,6 +255,8 @@ extern "C" int mi355x_moe_block_bwd(const mi355x_moe_block_bwd_args* a, void* st
       backward_space(a->workspace, a->tokens, h, i, a->experts, a->top_k, need_w13, need_w2,
                      a->grad_router != nullptr);
   MI355X_REQUIRE(a->workspace_bytes >= s.total, "moe_block_bwd: workspace too small");
+  MI355X_REQUIRE(((uintptr_t)a->workspace & 15) == 0,
+                 "moe_block_bwd: the workspace must be 16-byte aligned");
   const int padded = (int)mi355x_wgrad_padded_rows(rows, a->experts);
   STEP(mi355x_padded_row_blocks(a->offsets, a->experts, padded, s.blocks, stream));
   STEP(mi355x_swiglu_bwd_quantize(a->r, a->h13, a->route_weights, a->order, s.blocks, rows, i,

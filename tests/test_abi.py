@@ -56,6 +56,33 @@ def test_validation_errors(name, args, message):
         _native.call(name, *args)
 
 
+def _gemm_arguments(workspace, size):
+    # 4096 rows over 8 experts, N 4096, K 14336: a last round that may be split.
+    return _native.GEMM_ARGS.pack(*[0] * 10, workspace, size, 4096, 0, 1, 8, 4096, 14336, *[0] * 5)
+
+
+def _backward_arguments(workspace, size):
+    return _native.MOE_BLOCK_BWD_ARGS.pack(*[0] * 21, workspace, size, 16, 256, 128, 4, 2, 0, 1, 1,
+                                           0, 0.0)
+
+
+@pytest.mark.parametrize("name,args", [
+    ("mi355x_moe_route", lambda at, n: (None, 100, 8, 2, 0, None, 1, 1, 1.0, None, 1, None, None,
+                                        2, *[None] * 8, at, n, None)),
+    ("mi355x_moe_down", lambda at, n: (None, 16, 2, 256, 128, 0.0, 0, None, None, 4, *[None] * 5,
+                                       at, n, None)),
+    ("mi355x_moe_block_bwd", lambda at, n: (_backward_arguments(at, n), None)),
+    ("mi355x_gemm_fp8", lambda at, n: (_gemm_arguments(at, n), None)),
+])
+def test_workspaces_must_be_aligned(name, args):
+    """Every buffer of a sequence lies at 256-byte steps from its workspace and
+    takes 16-byte vector accesses."""
+    with pytest.raises(_native.NativeError, match="workspace must be 16-byte aligned"):
+        _native.call(name, *args(0x10008, 1 << 30))
+    with pytest.raises(_native.NativeError, match="workspace too small"):
+        _native.call(name, *args(0x10000, 16))
+
+
 def test_packed_argument_structs_cover_the_c_ones():
     """The entry points copy the whole struct, tail padding included."""
     assert _native.GEMM_ARGS.size == _native.query("mi355x_gemm_args_size")
