@@ -15,7 +15,7 @@ from dataclasses import dataclass
 from types import MappingProxyType
 
 from .context import implementation_override, record_dispatch
-from .registry import Implementation, SupportResult, frozen_implementation, implementations_for
+from .registry import Implementation, SupportResult, implementations_for
 
 SURFACES = ("semantic", "explicit")
 
@@ -88,15 +88,11 @@ def resolve_implementation(operation: str, *args, surface: str = "semantic",
             record_dispatch(str(operation), record.implementation_id)
             return record
     explanation = explain_implementation(operation, *args, surface=surface, **kwargs)
-    if explanation.selected is None:
-        refusals = "; ".join(f"{key}: {verdict.reason}"
-                             for key, verdict in sorted(explanation.candidates.items()))
-        what = ("no supported implementation" if explanation.forced is None
-                else f"the forced implementation {explanation.forced!r} does not support it")
-        raise RuntimeError(f"{what} for {explanation.operation!r} ({surface} surface): "
-                           f"{refusals}")
-    record_dispatch(explanation.operation, explanation.selected)
-    return frozen_implementation(explanation.operation, explanation.selected)
+    refusals = "; ".join(f"{key}: {verdict.reason}"
+                         for key, verdict in sorted(explanation.candidates.items()))
+    what = ("no supported implementation" if explanation.forced is None
+            else f"the forced implementation {explanation.forced!r} does not support it")
+    raise RuntimeError(f"{what} for {explanation.operation!r} ({surface} surface): {refusals}")
 
 
 def implementation_pairs(operations) -> Mapping[str, Mapping[str, Mapping[str, str]]]:
