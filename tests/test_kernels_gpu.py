@@ -474,6 +474,35 @@ TILE_CASES = [
 
 @pytest.mark.parametrize("counts,n,k", TILE_CASES)
 def test_grouped_gemm_forms_at_every_tile_size(device, counts, n, k):
+    _every_form(device, counts, n, k)
+
+
+# More tiles than the 2 x 256 workgroups of the 64- and 128-row tiles, so each
+# walks several: its issue pointer and its two gathered-row tables cross tile
+# borders, at K steps below, at and above the depth of the copy pipeline (3
+# stages for 64 rows, 2 for 128), experts of no rows among them.
+WALKED_64 = [(7 * e * e + 3) % 71 for e in range(24)] + [0]
+WALKED_128 = [129, 200, 256, 1, 250, 140, 0, 257, 129, 160]
+
+
+@pytest.mark.parametrize("tile,counts,n,k", [
+    (64, WALKED_64, 4096, 128),
+    (64, WALKED_64, 4096, 256),
+    (64, WALKED_64, 4096, 384),
+    (64, WALKED_64, 3072, 640),
+    (128, WALKED_128, 6144, 128),
+    (128, WALKED_128, 5120, 256),
+    (128, WALKED_128, 5120, 640),
+])
+def test_grouped_gemm_forms_over_several_tiles(device, tile, counts, n, k):
+    rows_per_expert = sum(counts) // len(counts)
+    assert rows_per_expert <= 48 if tile == 64 else 128 < rows_per_expert <= 160
+    tiles = sum(-(-c // tile) for c in counts) * (n // 128)
+    assert tiles > 2 * torch.cuda.get_device_properties(device).multi_processor_count
+    _every_form(device, counts, n, k)
+
+
+def _every_form(device, counts, n, k):
     """Every operand form at each tile size against the fp64 product of the
     dequantized operands. Bound: one bf16 rounding of the result is 2^-9 of
     each element, fp32 sums of K / 128 block partials add 1e-6, and a 128
@@ -875,7 +904,7 @@ def test_rowwise_gemm_large_weight_tile_order(device):
         assert max_rel(out[lo:hi].float(), want) < 1e-2, e
 
 
-# (256, 384): general kernel; (512, 768): the pipelined hardware-scaled one.
+# Both on the 128 x 128 tiles, (256, 384) outside the widths of the wide ones.
 @pytest.mark.parametrize("features", [(256, 384), (512, 768)])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_wgrad_matches_fp64(device, out_dtype, features):
@@ -904,6 +933,11 @@ def test_wgrad_matches_fp64(device, out_dtype, features):
     ([40, 300, 0, 257], (384, 640)),                   # several K blocks, an empty expert
     ([3] * 31 + [0], (1024, 512)),                     # 256 tiles of 256 x 256: the wide kernel
     ([130] * 7 + [0] * 18 + [1] * 7, (512, 1024)),
+    # Several tiles a workgroup (1440 on 512, 384 on 256), and with them the wait
+    # that leaves the last tile's stores in flight: experts of no rows at the
+    # start, in the middle and at the end, of one row and of many K blocks.
+    ([0, 1, 300, 129, 0, 0, 1, 700, 128, 1, 0, 513, 2, 40, 1, 0], (1280, 1152)),
+    ([0, 1, 300, 129, 0, 0, 1, 700, 128, 1, 0, 513, 2, 40, 1, 0], (1024, 1536)),
 ])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_wgrad_at_both_tile_sizes(device, out_dtype, counts, features):
