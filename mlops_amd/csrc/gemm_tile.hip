@@ -508,27 +508,50 @@ long long row_blocks(int rows, int groups, int bm) {
 Tiles choose_tiles(int rows, int experts, int n) {
   const int groups = rows < experts ? rows : experts;
   const int per_group = rows / groups, cus = cu_count();
-  // Measured on MI355X, weights from HBM, us (256 x 256 tiles of gemm_v2.hip
-  // / 128-row / 64-row tiles). 64-row tiles to 48 rows a group, where the
-  // launch is HBM-bound: hidden 2048, 2 x 768, 128 experts at 192 rows up
-  // 107 / 66 / 57, down 44 / 35 / 31 (6.1 and 5.6 TB/s of weights); at 4072
-  // rows 137 / 97 / 88 and 64 / 51 / 48.
+  // The loads are on the device, so the lines lie by their average. Measured on
+  // MI355X, weights from HBM, us (256 x 256 tiles of gemm_v2.hip / 128-row /
+  // 64-row tiles). With half of the rows on one expert, or loads after a Zipf
+  // law, no line loses to the 256 x 256 tiles; with all rows on one expert the
+  // 64-row tiles take 0.5 to 1.6 of their time (128 experts of hidden 2048, 768:
+  // 1024 rows up 30 / 16, 4096 rows 31 / 30, 6144 rows 33 / 44).
+  //
+  // 64-row tiles to 48 rows a group, where the launch is HBM-bound: hidden 2048,
+  // 2 x 768, 128 experts at 192 rows up 107 / 66 / 57, down 44 / 35 / 31 (6.1
+  // and 5.6 TB/s of weights); at 4072 rows 137 / 97 / 88 and 64 / 51 / 48.
   if (per_group <= 48) return Tiles::k64;
   // 128-row tiles that would leave CUs without a second workgroup keep too
   // little in flight: hidden 4096, 14336, 8 experts at 256 rows down
   // 187 / 118 / 86.
   if (per_group <= 128 && row_blocks(rows, groups, 128) * (n / TN) <= cus) return Tiles::k64;
-  // 128-row tiles to 160 rows a group (1024 a group of 128: up 164 / 143 /
-  // 165, down 81 / 76 / 91); from 192 on the 256 x 256 tile's reuse wins (176
-  // / 183 / 212 and 94 / 100 / 122).
+  if (n % 256 == 0) {
+    // A 256 x 256 grid that fills less than half the CUs: hidden 512, 1024, 8
+    // experts at 4096 rows, dx 33 / 21, down 19 / 13. Or just half of them, to
+    // 160 rows a group: hidden 1024, 2048, 8 experts at 640 rows up 16 / 13.
+    const long long wide = row_blocks(rows, groups, 256) * (n / 256);
+    if (2 * wide < cus || (2 * wide == cus && per_group <= 160)) return Tiles::k128;
+    // 128-row tiles to 64 rows a group where they make one and a half rounds of
+    // two workgroups a CU or more, so that an uneven routing's extra blocks are
+    // a small part. At 49 / 64 rows a group, uniform routing: hidden 7168, 2048, 32
+    // experts up 191, 196 / 173, 191; hidden 4096, 14336, 8 experts up 211, 209
+    // / 182, 192, gathered 236, 239 / 196, 215; hidden 2048, 768, 128 experts
+    // equal. One round of them (hidden 4096, 2048, 16 experts): row-scaled up
+    // 50 / 45 uniform, but 55 / 69 with experts of unequal load.
+    // Beyond, 256 x 256 tiles, whose waves past the expert's rows skip their
+    // work: an expert of 129 rows is one block of them and two of 128. 128
+    // experts of hidden 2048, 768 at 128 rows a group up 104 / 128, down 54 / 78,
+    // at 160 114 / 162 and 61 / 93. On uneven loads the two lie within 20% of
+    // each other, but where the wide grid just fills the CUs a block more is a
+    // round more (hidden 4096, 2048, 16 experts at 96 rows: down 25 / 30 even,
+    // 55 / 35 uneven). Over 2-200 rows a group of eight layer shapes, even,
+    // uniform and uneven, the lines never lose more than 5% to 256 x 256 tiles.
+    if (per_group <= 64 && row_blocks(rows, groups, 128) * (n / TN) >= 3ll * cus) return Tiles::k128;
+    return Tiles::kNone;
+  }
+  // N an odd multiple of 128 (no 256-column tile): 128-row tiles, from 161 rows
+  // a group on 256 x 128 tiles once they fill the CUs three times (hidden 1152,
+  // 640, 16 experts at 12004 rows: 36 us against 51; hidden 4096, 14336, 8
+  // experts at 4096 rows: 789 against 742).
   if (per_group <= 160) return Tiles::k128;
-  // A 256 x 256 grid that fills less than half the CUs: hidden 512, 1024, 8
-  // experts at 4096 rows, dx 33 / 21 / 23, down 19 / 13 / 14.
-  if (n % 256 == 0) return row_blocks(rows, groups, 256) * (n / 256) < cus / 2 ? Tiles::k128 : Tiles::kNone;
-  // N an odd multiple of 128 (no 256-column tile): 256 x 128 tiles once they
-  // fill the CUs three times, else 128-row tiles (hidden 1152, 640, 16
-  // experts at 12004 rows: 36 us against 51; hidden 4096, 14336, 8 experts at
-  // 4096 rows: 789 against 742).
   return row_blocks(rows, groups, 256) * (n / TN) >= 3ll * cus ? Tiles::k256 : Tiles::k128;
 }
 

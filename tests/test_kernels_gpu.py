@@ -455,8 +455,8 @@ def test_route_tokens_against_separate_calls(device, tokens, width, experts, top
 
 # Row counts and N that reach each tile size of the grouped GEMM: 64-row tiles
 # (few rows a group; 1 to 3 K steps, shorter than the copy pipeline), 128-row
-# tiles (129..160 rows a group), the 256 x 256 tiles, and 256 x 128 tiles (N an
-# odd multiple of 128 over many row blocks).
+# tiles (a 256 x 256 grid that fills less than half the CUs), the 256 x 256
+# tiles, and 256 x 128 tiles (N an odd multiple of 128 over many row blocks).
 TILE_CASES = [
     ([1, 63, 64, 65, 0, 17], 512, 128),
     ([1, 63, 64, 65, 0, 17], 768, 256),
@@ -482,7 +482,7 @@ def test_grouped_gemm_forms_at_every_tile_size(device, counts, n, k):
 # borders, at K steps below, at and above the depth of the copy pipeline (3
 # stages for 64 rows, 2 for 128), experts of no rows among them.
 WALKED_64 = [(7 * e * e + 3) % 71 for e in range(24)] + [0]
-WALKED_128 = [129, 200, 256, 1, 250, 140, 0, 257, 129, 160]
+WALKED_128 = [129, 10, 0, 256, 1, 9, 140, 0, 257, 30, 2, 127, 5, 0, 17, 33]
 
 
 @pytest.mark.parametrize("tile,counts,n,k", [
@@ -490,13 +490,13 @@ WALKED_128 = [129, 200, 256, 1, 250, 140, 0, 257, 129, 160]
     (64, WALKED_64, 4096, 256),
     (64, WALKED_64, 4096, 384),
     (64, WALKED_64, 3072, 640),
-    (128, WALKED_128, 6144, 128),
-    (128, WALKED_128, 5120, 256),
-    (128, WALKED_128, 5120, 640),
+    (128, WALKED_128, 8192, 128),
+    (128, WALKED_128, 8192, 256),
+    (128, WALKED_128, 8192, 384),
 ])
 def test_grouped_gemm_forms_over_several_tiles(device, tile, counts, n, k):
     rows_per_expert = sum(counts) // len(counts)
-    assert rows_per_expert <= 48 if tile == 64 else 128 < rows_per_expert <= 160
+    assert rows_per_expert <= 48 if tile == 64 else 48 < rows_per_expert <= 64
     tiles = sum(-(-c // tile) for c in counts) * (n // 128)
     assert tiles > 2 * torch.cuda.get_device_properties(device).multi_processor_count
     _every_form(device, counts, n, k)
@@ -559,7 +559,7 @@ def _every_form(device, counts, n, k):
     ([1, 63, 64, 65, 0, 300, 17], 4096, 128, 2304),   # 64-row tiles; nk = 1
     ([1, 63, 64, 65, 0, 300, 17], 4096, 384, 2304),   # nk < 8: the full rotation
     ([1, 63, 64, 65, 0, 300, 17], 4096, 1024, 2304),  # nk >= 8: three starts
-    ([1, 63, 64, 65, 0, 300, 17], 6400, 4096, 2304),  # the large weight's order: no rotation
+    ([1, 63, 64, 65, 0, 300, 17], 4096, 6144, 2304),  # the large weight's order: no rotation
     ([129, 600, 1, 0, 70], 4096, 640, 2304),          # 128-row tiles
     ([500, 520, 500, 530, 0, 510, 1, 515], 512, 1152, 16384),  # wide grid too small
 ])
@@ -686,6 +686,7 @@ def test_grouped_gemm_last_round_split_over_k(device, monkeypatch, counts, n, k)
     (2048, 8, 4096, 14336, False),   # 24 expected, 22 to 26 likely: no half-empty round
     (16384, 32, 7168, 2048, False),  # K too short to split
     (640, 8, 4096, 14336, False),    # smaller tiles
+    (2304, 16, 4096, 8192, True),    # 144 rows an expert: wide ones, 2 of 34 an XCD left over
     (0, 8, 4096, 14336, False),
 ])
 def test_gemm_tail_workspace_where_a_short_last_round_is_likely(device, rows, experts, n, k,
