@@ -12,8 +12,8 @@
 // K block) at the granularity the hardware gives for free.
 //
 // MFMA operand layout (verified on MI355X): lane l supplies row l%16 of A
-// and column l%16 of B, each as 32 consecutive K bytes starting at
-// 32*(l/16); the 4 outputs of lane l are rows 4*(l/16)+i, column l%16.
+// and column l%16 of B, each as the K bytes 16g..16g+15 and 64+16g..64+16g+15
+// with g = l/16; its 4 outputs are rows 4g+i, column l%16.
 #include "common.h"
 
 namespace {
@@ -66,9 +66,9 @@ mi355x_gemm_args operands(const uint8_t* a, const float* a_scale, int rows, cons
 
 // Gathered-A forms: GEMM row r (expert-sorted, offsets) reads row
 // a_rows[r] of a [a_total, K] and its 1x128 scales a_scale[a_total][K/128]
-// (token-major, as mi355x_quantize_token_rows_fp8 writes them)
-// (the activation quantized once per token; a_rows = the token of each
-// routed row). Pipelined kernel only (N a multiple of 256).
+// (token-major, as mi355x_quantize_token_rows_fp8 writes them): the activation
+// quantized once per token, a_rows / a_rows_div the token of each routed row.
+// N a multiple of 256, on the 256 x 256 tiles or the smaller ones.
 int gathered_checks(const mi355x_gemm_args& g) {
   MI355X_REQUIRE(g.a_rows != nullptr && g.a_total > 0, "gemm gathered: a_rows and a_total required");
   MI355X_REQUIRE(g.a_rows_div >= 1 && (uint64_t)g.a_total * (uint64_t)g.a_rows_div < (1ull << 31),

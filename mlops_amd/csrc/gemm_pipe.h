@@ -188,12 +188,9 @@ __device__ __forceinline__ int find_expert(const int* prefix, int experts, int t
   return lo;
 }
 
-// Persistent tile order: in each round of G tiles, XCD x (= block % 8) takes
-// the G/8 consecutive tiles starting at x * G/8, so the 32 CUs of one XCD
-// share A rows across N tiles and weights across M tiles in their L2.
-// Round-robin tile assignment. Grouping consecutive tiles onto one XCD (block
-// b runs on XCD b % 8) raised the L2 hit rate from ~10% to ~64% but measured
-// 5-20% slower on the MoE and dense shapes, so tiles go out in plain order.
+// Round-robin tile assignment, for grids that are no multiple of 8 workgroups.
+// The others give XCD x (= workgroup % 8) the x-th eighth of the tile list, so
+// that its CUs share panels in their L2 (tile_at in each kernel).
 __device__ __forceinline__ int tile_of(int round, int block, int grid) {
   return round * grid + block;
 }

@@ -25,7 +25,7 @@ constexpr int kMaxExperts = 512;
 // eight consecutive bf16 columns (one 16-byte store); with fp32 outputs
 // columns 4c .. 4c + 3 of either half, so that each of the two 16-byte
 // stores of a row fills whole lines (32 bytes per lane, stored as two halves
-// of a line, took 930 us for 1.6 GB of gradients where this takes 271).
+// of a line, took 930 us for 1.6 GB of gradients where this takes 269).
 template <bool kFp32>
 __device__ __forceinline__ int feature_col(int tr, int nt) {
   const int part = tr >> 7, local = tr & 127, c = local & 15, jb = local >> 4;

@@ -51,8 +51,8 @@ struct Raw<float> {
 template <typename W>
 __global__ void __launch_bounds__(64 * kLogitWaves) router_logits_kernel(
     const uint16_t* __restrict__ x, const W* __restrict__ weight, int tokens, int experts,
-    int width, int chunks, int blocks, float* __restrict__ partial, int pitch, int quantize, uint8_t* __restrict__ q,
-    float* __restrict__ scales) {
+    int width, int chunks, int blocks, float* __restrict__ partial, int pitch, int quantize,
+    uint8_t* __restrict__ q, float* __restrict__ scales) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = lane_id();
   if ((int)blockIdx.x >= blocks) {
     const int r = (blockIdx.x - blocks) * kLogitWaves + wave;

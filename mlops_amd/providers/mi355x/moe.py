@@ -5,11 +5,12 @@ Registered behind the same registry contract as the reference providers
 fakes, autograd and FLOP formulas; ``providers/sonicmoe/moe.py:441-620`` and
 ``providers/sonicmoe/block_fp8.py`` for the block-FP8 math it serves). Every
 step from the fp32 router logits on is a hand-written HIP kernel of
-``libmlops_mi355x.so``; the router GEMM and its two small gradient GEMMs stay on
-hipBLASLt through torch, as the reference keeps them on cuBLAS.
+``libmlops_mi355x.so``. The router GEMM is one too up to 64 tokens, and its
+weight gradient from 64 experts up; else they and the router's input gradient
+run on hipBLASLt through torch, as the reference keeps them on cuBLAS.
 
 Forward (sorted rows ``A = T * k``):
-  logits = bf16 x @ bf16 Wr^T (fp32)          router GEMM
+  logits = bf16 x @ bf16 Wr^T (fp32)          router GEMM (<= 64 tokens: with the next two)
   weights, ids = router_topk(logits)          one wave per token
   counts, offsets, order, slots = plan(ids)   stable counting sort
   xq = quantize_rows(x)                       e4m3 token rows (1x128); k < 4: permuted

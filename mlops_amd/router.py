@@ -10,8 +10,10 @@ Semantics of ``src/mlops/kernels/router.py:54-113`` on the GPU:
   each multiplied against the bf16 activation with fp32 sums (fp32-quality
   gradient for an fp32 master), then written at the requested dtype.
 
-These small GEMMs ([T,H]x[H,E]) run on hipBLASLt through torch; the MoE
-provider's own kernels take over from the fp32 logits.
+These small GEMMs ([T,H]x[H,E]) run on hipBLASLt through torch, but for the
+logits of few tokens (``kernels.route_tokens``) and the weight gradient of many
+experts (``kernels.router_weight_grad``); the MoE provider's own kernels take
+over from the fp32 logits.
 """
 
 from __future__ import annotations

@@ -1,5 +1,5 @@
 """The gathered GEMMs read token order[r] // top_k through a multiply-high
-division by an invariant divisor (csrc/gemm_v2.hip: row_div_magic on the
+division by an invariant divisor (csrc/gemm_pipe.h: row_div_magic on the
 host, div_rows in the kernel; the round-down method of Granlund and
 Montgomery, PLDI 1994, with a 33-bit multiplier). This checks the method's
 constants and steps against exact integer division on the CPU: every x below
